@@ -317,23 +317,19 @@ int mk_gemm(int in_type, int epi, const void* A, int lda, const void* B, int ldb
 
 int mk_lm_head(const void* hidden, const void* lm_head, int B, int H, int V, float* logits, void* stream) {
   MK_REQUIRE(hidden && lm_head && logits && B >= 1 && H >= 1 && V >= 1, "lm_head: bad arguments");
-  for (int b0 = 0; b0 < B; b0 += 32) {
-    mk::GemmArgs g{};
-    g.in = mk::GemmIn::BF16;
-    g.epi = mk::Epi::F32;
-    g.A = static_cast<const uint16_t*>(hidden) + (size_t)b0 * H;
-    g.lda = H;
-    g.B = lm_head;
-    g.ldb = H;
-    g.M = B - b0 < 32 ? B - b0 : 32;
-    g.N = V;
-    g.K = H;
-    g.out = logits + (size_t)b0 * V;
-    g.ldo = V;
-    int rc = mk::launch_gemm_skinny(g, static_cast<hipStream_t>(stream));
-    if (rc) return rc;
-  }
-  return MK_OK;
+  mk::GemmArgs g{};
+  g.in = mk::GemmIn::BF16;
+  g.epi = mk::Epi::F32;
+  g.A = hidden;
+  g.lda = H;
+  g.B = lm_head;
+  g.ldb = H;
+  g.M = B;
+  g.N = V;
+  g.K = H;
+  g.out = logits;
+  g.ldo = V;
+  MK_TRY(mk::launch_lm_head(g, static_cast<hipStream_t>(stream)));
 }
 
 int mk_pack_weight(const void* in, int ld_in, void* out, int K, int N, int elem_bytes, int map, int ic, int inter,

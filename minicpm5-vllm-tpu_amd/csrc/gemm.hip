@@ -935,6 +935,89 @@ __global__ __launch_bounds__(64 * SK_WAVES) void gemm_skinny16_kernel(GemmArgs g
   }
 }
 
+// LM head: up to 64 rows of A against each weight row in one pass over the weights.  The weight stream
+// (V x H bf16, 400 - 535 MB) is the bound, so it must be read once, with enough of it in flight.  The skinny
+// kernel takes 32 rows at a time, so above 32 it read the weights twice, and each of its waves reads all of
+// A from L2 for its 16 columns.  Here the 8 waves of a workgroup (16 columns each) share A: chunks of 256 k
+// are copied to LDS, two buffers, and each wave keeps the next chunk's 8 weight loads (8 KB) in flight while
+// it multiplies the current one, with two or more workgroups per CU.  Measured at V = 130560, us, H = 1536 /
+// 2048, skinny kernel then this one: 1 row 73.0 / 93.4 -> 68.4 / 96.5, 8 rows 85.4 / 106.9 -> 73.2 / 98.6,
+// 32 rows 135.3 / 176.6 -> 85.9 / 109.1, 40 rows 220 -> 88.5 (4.5 TB/s) at H = 1536.  The MFMAs of an output
+// element are the skinny kernel's in the same order, so a row's logits do not depend on the batch size.
+constexpr int LH_WAVES = 8, LH_KB = 512;   // waves per workgroup, bytes of K per chunk
+
+template <int MG>   // groups of 16 rows
+__global__ __launch_bounds__(64 * LH_WAVES) void lm_head_kernel(GemmArgs g) {
+  constexpr int ROWS = 16 * MG, BUF = ROWS * LH_KB, QA = BUF / 1024 / LH_WAVES;
+  static_assert(QA >= 1 && QA * LH_WAVES * 1024 == BUF, "A copies split evenly over the waves");
+  __shared__ __attribute__((aligned(1024))) char smem[2 * BUF];
+  const int lane = threadIdx.x & 63;
+  const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int c16 = lane & 15, kg = lane >> 4;
+  const int n0 = (blockIdx.x * LH_WAVES + w) * 16;
+  const int lda = g.lda * 2, ldb = g.ldb * 2;
+  const __amdgpu_buffer_rsrc_t rA = make_rsrc(g.A, (uint32_t)((size_t)g.M * lda));
+  // A copy j of this wave: rows 2 (w + 8 j) and the next, 512 bytes each; 16-byte chunk c of row r sits at
+  // slot c ^ (r % 16), so the 16 rows a phase of the operand reads covers fall on distinct banks.  Rows past
+  // M repeat the last one (never stored).
+  uint32_t aoff[QA];
+#pragma unroll
+  for (int j = 0; j < QA; ++j) {
+    const int r = 2 * (w + LH_WAVES * j) + (lane >> 5);
+    aoff[j] = (uint32_t)min(r, g.M - 1) * (uint32_t)lda + 16u * ((lane & 31) ^ (r & 15));
+  }
+  auto copy_a = [&](int buf, int kb) {
+#pragma unroll
+    for (int j = 0; j < QA; ++j)
+      copy16_to_lds(rA, aoff[j], (uint32_t)kb, smem + buf * BUF + (w + LH_WAVES * j) * 1024);
+  };
+  const char* bp = static_cast<const char*>(g.B) + (size_t)min(n0 + c16, g.N - 1) * ldb + kg * 16;
+  auto load_b = [&](u32x4 (&b)[8], int kb) {
+#pragma unroll
+    for (int u = 0; u < 8; ++u) b[u] = *reinterpret_cast<const u32x4*>(bp + kb + 64 * u);
+  };
+  f32x4 acc[MG];
+#pragma unroll
+  for (int i = 0; i < MG; ++i) acc[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+  u32x4 b0[8], b1[8];
+  const int nc = g.K * 2 / LH_KB;
+  copy_a(0, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  load_b(b0, 0);
+  __builtin_amdgcn_sched_barrier(0);
+  auto chunk = [&](int c, u32x4 (&b)[8], u32x4 (&bn)[8]) {
+    MK_WAIT_VMCNT(8);                       // A(c) landed; the 8 loads of b may be in flight
+    __builtin_amdgcn_s_waitcnt(0xc07f);     // this wave's reads of A(c - 1) are done
+    lds_barrier();
+    if (c + 1 < nc) {
+      copy_a((c + 1) & 1, (c + 1) * LH_KB);
+      __builtin_amdgcn_sched_barrier(0);    // the copies stay ahead of the weight loads (vmcnt order)
+      load_b(bn, (c + 1) * LH_KB);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const char* S = smem + (c & 1) * BUF + c16 * LH_KB;
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+#pragma unroll
+      for (int i = 0; i < MG; ++i)
+        acc[i] = mfma_bf16_16x16x32(
+            *reinterpret_cast<const u32x4*>(S + i * 16 * LH_KB + 16 * ((4 * u + kg) ^ c16)), b[u], acc[i]);
+  };
+  for (int c = 0; c < nc; c += 2) {
+    chunk(c, b0, b1);
+    if (c + 1 < nc) chunk(c + 1, b1, b0);
+  }
+  const int n = n0 + c16;
+  if (n >= g.N) return;
+#pragma unroll
+  for (int i = 0; i < MG; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int m = 16 * i + 4 * kg + j;
+      if (m < g.M) static_cast<float*>(g.out)[(size_t)m * g.ldo + n] = acc[i][j];
+    }
+}
+
 // Sum of the split-K partials in split order, then the epilogue.
 // Every partial is loaded before the first add (one memory latency, not one per group of loads).
 constexpr int SK_MAX_SPLITS = 16;
@@ -1223,6 +1306,37 @@ int launch_gemm_skinny(const GemmArgs& g, hipStream_t st) {
     case GemmIn::F8: return dispatch<GemmIn::F8>(g, st, true);
     default: return dispatch<GemmIn::BF16>(g, st, true);
   }
+}
+
+int launch_lm_head(const GemmArgs& g0, hipStream_t st) {
+  // Up to 64 rows per pass.  The batch kernel takes whole 512-byte K chunks; a single row over more than
+  // three of them is faster on the skinny kernel, which has no barriers to pay for (measured above).
+  const bool whole = g0.K > 0 && g0.K * 2 % LH_KB == 0;
+  const int lo = whole && g0.K * 2 <= 3 * LH_KB ? 0 : 1;
+  for (int m0 = 0, rows; m0 < g0.M; m0 += rows) {
+    GemmArgs g = g0;
+    const int left = g0.M - m0;
+    g.A = static_cast<const uint16_t*>(g0.A) + (size_t)m0 * g0.lda;
+    g.out = static_cast<float*>(g0.out) + (size_t)m0 * g0.ldo;
+    if (!whole || left <= lo) {
+      rows = g.M = std::min(32, left);
+      const int rc = launch_gemm_skinny(g, st);
+      if (rc) return rc;
+      continue;
+    }
+    rows = g.M = std::min(64, left);
+    const int rc = gemm_validate(g);
+    if (rc) return rc;
+    const dim3 grid((g.N + 16 * LH_WAVES - 1) / (16 * LH_WAVES)), block(64 * LH_WAVES);
+    switch ((rows + 15) / 16) {
+      case 1: hipLaunchKernelGGL((lm_head_kernel<1>), grid, block, 0, st, g); break;
+      case 2: hipLaunchKernelGGL((lm_head_kernel<2>), grid, block, 0, st, g); break;
+      case 3: hipLaunchKernelGGL((lm_head_kernel<3>), grid, block, 0, st, g); break;
+      default: hipLaunchKernelGGL((lm_head_kernel<4>), grid, block, 0, st, g); break;
+    }
+    MK_HIP_CHECK(hipGetLastError());
+  }
+  return MK_OK;
 }
 
 }  // namespace mk

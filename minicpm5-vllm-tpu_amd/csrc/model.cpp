@@ -717,22 +717,19 @@ int launch_forward(const Fwd& f, hipStream_t st) {
   MK_RUN(launch_rmsnorm_bf16(xl, H, static_cast<const uint16_t*>(m.w.final_norm), f.hidden, H, B, H, c.eps, st));
   kind = MK_KERNEL_LM_HEAD;
   if (f.logits) {
-    for (int b0 = 0; b0 < B; b0 += 32) {
-      const int rows = std::min(32, B - b0);
-      GemmArgs g{};
-      g.in = GemmIn::BF16;
-      g.epi = Epi::F32;
-      g.M = rows;
-      g.K = H;
-      g.N = c.vocab;
-      g.A = f.hidden + (size_t)b0 * H;
-      g.lda = H;
-      g.B = m.w.lm_head;
-      g.ldb = H;
-      g.out = f.logits + (size_t)b0 * c.vocab;
-      g.ldo = c.vocab;
-      MK_RUN(launch_gemm_skinny(g, st));
-    }
+    GemmArgs g{};
+    g.in = GemmIn::BF16;
+    g.epi = Epi::F32;
+    g.M = B;
+    g.K = H;
+    g.N = c.vocab;
+    g.A = f.hidden;
+    g.lda = H;
+    g.B = m.w.lm_head;
+    g.ldb = H;
+    g.out = f.logits;
+    g.ldo = c.vocab;
+    MK_RUN(launch_lm_head(g, st));
   }
 #undef MK_RUN
   return MK_OK;

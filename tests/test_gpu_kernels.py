@@ -424,6 +424,27 @@ def _pack_gu_scales(s_il, inter):
     return s_il.reshape(-1)[src].contiguous()
 
 
+@pytest.mark.parametrize("V,H", [(1000, 1536), (1000, 2048), (520, 256), (520, 1152)])
+def test_lm_head_batches(V, H):
+    """Batches at the edges of the LM head's 16-row groups and 64-row passes (H = 1152: no whole 256-element
+    chunks, the 32-row kernel): f32 sums of exact bf16 products, so each logit is within 32 eps sum|products|
+    of the float64 one, and a row's bits do not depend on the batch."""
+    from minicpm5_mk import ops
+
+    dev = _dev()
+    g = torch.Generator().manual_seed(V + H)
+    x = torch.randn(129, H, generator=g).to(BF16).to(dev)
+    w = (torch.randn(V, H, generator=g) * 0.02).to(BF16).to(dev)
+    full = ops.lm_head(x, w)
+    ref = x.double() @ w.double().t()
+    bound = 32 * 2.0 ** -24 * (x.double().abs() @ w.double().abs().t())
+    for B in (1, 2, 15, 16, 17, 32, 33, 48, 49, 64, 65, 80, 128):
+        out = ops.lm_head(x[:B].contiguous(), w)
+        assert ((out.double() - ref[:B]).abs() <= bound[:B]).all(), B
+        # a single row over more than 768 k takes the skinny kernel: same sums, same bits
+        assert torch.equal(out.view(torch.int32), full[:B].view(torch.int32)), B
+
+
 @pytest.mark.parametrize("smooth", [False, True])
 def test_decoder_block_int8(smooth):
     """Quantised decoder block at its full size (8192 tokens, MiniCPM5-1B hd-96 shapes): fused RMSNorm +

@@ -5,8 +5,11 @@
 // lane of a 32x32 MFMA reads 16 contiguous bytes of K for its row / column.
 //
 // int8 (v_mfma_i32_32x32x32_i8, exact int32 accumulation), bf16 (v_mfma_f32_32x32x16_bf16, f32
-// accumulation) and fp8 e4m3 (two v_mfma_f32_32x32x16_fp8_fp8, f32 accumulation) share one kernel:
-// each consumes 16 bytes of K per lane per k-step.
+// accumulation) and fp8 e4m3 (v_mfma_f32_32x32x64_f8f6f4, f32 accumulation) share one kernel: int8 and bf16
+// consume 16 bytes of K per lane per MFMA, fp8 32 (the whole 64-byte stage slice in one k-step, at twice
+// the rate of the K = 16 fp8 instruction; against float64 its sums are off by the same 1.5e-5 in 2-norm and
+// 1.5 - 3.8e-6 of sum|products| at K = 1536 .. 6144, M = 64 .. 4096).  2B gate/up at M = 4096: 144 -> 103 us,
+// QKV 39 -> 29 us.
 //
 // Epilogues restate the reference's dequant / activation / residual algebra exactly:
 //   fused_qkv      mk_mlp.py:169-170   out = bf16((acc * sx) * s_w)
@@ -99,6 +102,7 @@ struct Mma<GemmIn::I8> {
   using Elem = int;
   using Vec4 = i32x4;
   static constexpr int ESZ = 1;
+  static constexpr bool WIDE = false;   // one MFMA per 16 bytes of K
   __device__ static Acc run(const u32x4& a, const u32x4& b, const Acc& c) { return mfma_i8_32x32x32(a, b, c); }
   __device__ static float f(int v) { return static_cast<float>(v); }
 };
@@ -108,6 +112,7 @@ struct Mma<GemmIn::F8> {
   using Elem = float;
   using Vec4 = f32x4;
   static constexpr int ESZ = 1;
+  static constexpr bool WIDE = true;    // one MFMA per 32 bytes of K: a stage is one k-step (run: skinny kernel)
   __device__ static Acc run(const u32x4& a, const u32x4& b, const Acc& c) { return mfma_fp8_32x32x32(a, b, c); }
   __device__ static float f(float v) { return v; }
 };
@@ -117,6 +122,7 @@ struct Mma<GemmIn::BF16> {
   using Elem = float;
   using Vec4 = f32x4;
   static constexpr int ESZ = 2;
+  static constexpr bool WIDE = false;
   __device__ static Acc run(const u32x4& a, const u32x4& b, const Acc& c) { return mfma_bf16_32x32x16(a, b, c); }
   __device__ static float f(float v) { return v; }
 };
@@ -227,8 +233,9 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kernel(GemmArgs g) {
   // lane offset only).  The empty asm keeps the sum from being hoisted out of the loop into a register
   // of its own.
   const uint32_t lim_a = (uint32_t)(g.M - 1) * (uint32_t)lda + 48u, lim_b = (uint32_t)(g.N - 1) * (uint32_t)ldb + 48u;
+  constexpr bool LEAN = C::LEAN || (T::WIDE && C::LOOP == 1 && 16 * C::MT * C::NTL + 16 * (C::MT + C::NTL) > 216);
   auto voff = [&](int j) -> uint32_t {
-    if constexpr (!C::LEAN) {
+    if constexpr (!LEAN) {
       return loff[j];
     } else {
       const bool isa = j < JA;
@@ -283,6 +290,12 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kernel(GemmArgs g) {
   auto mf = [&](int i, const u32x4 (&ra)[C::MT], const u32x4 (&rb)[C::NTL]) {
     const int mt = i / C::NTL, nt = i % C::NTL;
     acc[mt][nt] = T::run(ra[mt], rb[nt], acc[mt][nt]);
+  };
+  // MFMA i of a whole stage (WIDE operand types): both 16-byte halves at once
+  auto mfw = [&](int i, const u32x4 (&ra0)[C::MT], const u32x4 (&rb0)[C::NTL], const u32x4 (&ra1)[C::MT],
+                 const u32x4 (&rb1)[C::NTL]) {
+    const int mt = i / C::NTL, nt = i % C::NTL;
+    if constexpr (T::WIDE) acc[mt][nt] = mfma_fp8_32x32x64(ra0[mt], ra1[mt], rb0[nt], rb1[nt], acc[mt][nt]);
   };
 
   // Software pipeline over the LDS ring (stage = BKB bytes of K = two MFMA k-steps):
@@ -368,6 +381,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kernel(GemmArgs g) {
     constexpr int D = C::NST - 1;
     constexpr int NOP = C::MT + C::NTL;                   // operand registers per k-step: B then A
     u32x4 H0[NOP], H1[NOP], H2[NOP];
+    u32x4 H3[T::WIDE ? NOP : 1];   // WIDE: stage s uses sets (H0, H1) or (H2, H3), all of a stage at once
     auto rdq = [&](const char* Sb, int ks, int q, u32x4 (&dst)[NOP]) {
       if (q < C::NTL) dst[q] = *reinterpret_cast<const u32x4*>(Sb + (ks ? bo1 : bo0) + q * 32 * BKB);
       else dst[q] = *reinterpret_cast<const u32x4*>(Sb + (ks ? ao1 : ao0) + (q - C::NTL) * 32 * BKB);
@@ -375,6 +389,11 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kernel(GemmArgs g) {
     auto mfq = [&](int i, const u32x4 (&src)[NOP]) {
       const int mt = i / C::NTL, nt = i % C::NTL;
       acc[mt][nt] = T::run(src[C::NTL + mt], src[nt], acc[mt][nt]);
+    };
+    auto mfqw = [&](int i, const u32x4 (&s0)[NOP], const u32x4 (&s1)[NOP]) {
+      const int mt = i / C::NTL, nt = i % C::NTL;
+      if constexpr (T::WIDE)
+        acc[mt][nt] = mfma_fp8_32x32x64(s0[C::NTL + mt], s1[C::NTL + mt], s0[nt], s1[nt], acc[mt][nt]);
     };
     // stages 0 and 1 visible; stage 0 in H0 / H1
     if (nk >= D) wait_stages(std::integral_constant<int, D - 2>{});
@@ -392,7 +411,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kernel(GemmArgs g) {
     int cur = 0;
     // `steady` instances (stage it + D exists) have no runtime conditions, so the compute phase stays one
     // basic block instead of a branch around every operand read
-    auto step = [&](auto steady, int it, u32x4 (&ha)[NOP], u32x4 (&hb)[NOP], u32x4 (&hc)[NOP]) {
+    auto step = [&](auto steady, int it, u32x4 (&ha)[NOP], u32x4 (&hb)[NOP], u32x4 (&hc)[NOP], u32x4 (&hd)[NOP]) {
       constexpr bool ST = decltype(steady)::value;
       // M(it): async loads of stage it + D into the slot of stage it - 1
       const bool pre = ST || it + D < nk;
@@ -411,24 +430,36 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kernel(GemmArgs g) {
       const char* S1 = smem + s1 * C::ST_BYTES;
       const bool nxt = ST || it + 1 < nk;
       __builtin_amdgcn_s_setprio(1);
+      if constexpr (T::WIDE) {
+        constexpr int NRD = 2 * NOP, RPM = (NRD + NMF - 1) / NMF;   // operand reads per MFMA
 #pragma unroll
-      for (int i = 0; i < NMF; ++i) {
-        mfq(i, ha);
-        if (i < NOP && nxt) rdq(S1, 0, i, hc);
-        __builtin_amdgcn_sched_barrier(0);
+        for (int i = 0; i < NMF; ++i) {
+          mfqw(i, ha, hb);
+#pragma unroll
+          for (int q = i * RPM; q < (i + 1) * RPM && q < NRD; ++q)
+            if (nxt) rdq(S1, q & 1, q >> 1, q & 1 ? hd : hc);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < NMF; ++i) {
+          mfq(i, ha);
+          if (i < NOP && nxt) rdq(S1, 0, i, hc);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int q = NMF; q < NOP; ++q)
+          if (nxt) rdq(S1, 0, q, hc);
+#pragma unroll
+        for (int i = 0; i < NMF; ++i) {
+          mfq(i, hb);
+          if (i < NOP && nxt) rdq(S1, 1, i, ha);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int q = NMF; q < NOP; ++q)
+          if (nxt) rdq(S1, 1, q, ha);
       }
-#pragma unroll
-      for (int q = NMF; q < NOP; ++q)
-        if (nxt) rdq(S1, 0, q, hc);
-#pragma unroll
-      for (int i = 0; i < NMF; ++i) {
-        mfq(i, hb);
-        if (i < NOP && nxt) rdq(S1, 1, i, ha);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-#pragma unroll
-      for (int q = NMF; q < NOP; ++q)
-        if (nxt) rdq(S1, 1, q, ha);
       __builtin_amdgcn_s_setprio(0);
       __builtin_amdgcn_s_waitcnt(0xc07f);                 // lgkmcnt(0): stage it + 1 is in registers
       if (wgrp == 1 && (ST || it + 2 < nk)) {
@@ -441,15 +472,26 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kernel(GemmArgs g) {
     using Steady = std::integral_constant<bool, true>;
     using Tail = std::integral_constant<bool, false>;
     int it = 0;
-    for (; it + 2 + D < nk; it += 3) {
-      step(Steady{}, it, H0, H1, H2);
-      step(Steady{}, it + 1, H2, H0, H1);
-      step(Steady{}, it + 2, H1, H2, H0);
-    }
-    for (; it < nk; it += 3) {
-      step(Tail{}, it, H0, H1, H2);
-      if (it + 1 < nk) step(Tail{}, it + 1, H2, H0, H1);
-      if (it + 2 < nk) step(Tail{}, it + 2, H1, H2, H0);
+    if constexpr (T::WIDE) {
+      for (; it + 1 + D < nk; it += 2) {
+        step(Steady{}, it, H0, H1, H2, H3);
+        step(Steady{}, it + 1, H2, H3, H0, H1);
+      }
+      for (; it < nk; it += 2) {
+        step(Tail{}, it, H0, H1, H2, H3);
+        if (it + 1 < nk) step(Tail{}, it + 1, H2, H3, H0, H1);
+      }
+    } else {
+      for (; it + 2 + D < nk; it += 3) {
+        step(Steady{}, it, H0, H1, H2, H2);
+        step(Steady{}, it + 1, H2, H0, H1, H1);
+        step(Steady{}, it + 2, H1, H2, H0, H0);
+      }
+      for (; it < nk; it += 3) {
+        step(Tail{}, it, H0, H1, H2, H2);
+        if (it + 1 < nk) step(Tail{}, it + 1, H2, H0, H1, H1);
+        if (it + 2 < nk) step(Tail{}, it + 2, H1, H2, H0, H0);
+      }
     }
     if (wgrp == 0) lds_barrier();
   } else if constexpr (C::LOOP == 2) {
@@ -478,7 +520,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kernel(GemmArgs g) {
       __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
       for (int i = 0; i < NMF; ++i) {
-        mf(i, xa0, xb0);
+        if constexpr (T::WIDE) mfw(i, xa0, xb0, xa1, xb1);
+        else mf(i, xa0, xb0);
         if (i < Q && pre0) issue1(i, ns0, (it + C::NST - 2) * BKB);
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -488,7 +531,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kernel(GemmArgs g) {
       }
 #pragma unroll
       for (int i = 0; i < NMF; ++i) {
-        mf(i, xa1, xb1);
+        if constexpr (!T::WIDE) mf(i, xa1, xb1);
         if (i < Q && pre1) issue1(i, ns1, (it + C::NST - 1) * BKB);
         __builtin_amdgcn_sched_barrier(0);
       }
@@ -496,7 +539,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kernel(GemmArgs g) {
 #pragma unroll
         for (int j = NMF; j < Q; ++j) issue1(j, ns1, (it + C::NST - 1) * BKB);
       }
-      if (two) {
+      if (!T::WIDE && two) {
 #pragma unroll
         for (int i = 0; i < NMF; ++i) {
           mf(i, xa2, xb2);
@@ -519,7 +562,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kernel(GemmArgs g) {
       if (two) {
 #pragma unroll
         for (int i = 0; i < NMF; ++i) {
-          mf(i, xa3, xb3);
+          if constexpr (T::WIDE) mfw(i, xa2, xb2, xa3, xb3);
+          else mf(i, xa3, xb3);
           __builtin_amdgcn_sched_barrier(0);
         }
       }
@@ -530,6 +574,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kernel(GemmArgs g) {
   } else {
     u32x4 ra0[C::MT], rb0[C::NTL], ra1[C::MT], rb1[C::NTL];
     rd(smem, ao0, bo0, ra0, rb0);
+    if constexpr (T::WIDE) rd(smem, ao1, bo1, ra1, rb1);
     int cur = 0;                                            // stage slot of iteration it
     constexpr int SPLIT = NMF / 4;                          // k-step 1 MFMAs issued before the barrier
     auto iter = [&](auto steady, int it) {
@@ -570,8 +615,41 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kernel(GemmArgs g) {
       __builtin_amdgcn_sched_barrier(0);
     };
     int it = 0;
-    for (; it + C::NST - 1 < nk; ++it) iter(std::integral_constant<bool, true>{}, it);
-    for (; it < nk; ++it) iter(std::integral_constant<bool, false>{}, it);
+    if constexpr (T::WIDE) {
+      // One k-step per stage: its MFMAs interleaved with the async loads, then the wait for stage it + 1, the
+      // barrier and that stage's operand reads; two resident workgroups per CU cover each other's reads.
+      auto iterw = [&](auto steady, int it) {
+        constexpr bool ST = decltype(steady)::value;
+        const bool pre = ST || it + C::NST - 1 < nk;
+        const int nslot = cur == 0 ? C::NST - 1 : cur - 1;
+        const int nkb = (it + C::NST - 1) * BKB;
+#pragma unroll
+        for (int i = 0; i < NMF; ++i) {
+          mfw(i, ra0, rb0, ra1, rb1);
+          if (i < Q && pre) issue1(i, nslot, nkb);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+        if (Q > NMF && pre) {
+#pragma unroll
+          for (int j = NMF; j < Q; ++j) issue1(j, nslot, nkb);
+        }
+        cur = cur == C::NST - 1 ? 0 : cur + 1;
+        if (ST || it + 1 < nk) {
+          if (pre) MK_WAIT_VMCNT((C::NST - 2) * Q);
+          else MK_WAIT_VMCNT(0);
+          __builtin_amdgcn_s_waitcnt(0xc07f);   // this wave's reads of stage it are done before its slot is refilled
+          lds_barrier();
+          rd(smem + cur * C::ST_BYTES, ao0, bo0, ra0, rb0);
+          rd(smem + cur * C::ST_BYTES, ao1, bo1, ra1, rb1);
+        }
+        __builtin_amdgcn_sched_barrier(0);
+      };
+      for (; it + C::NST - 1 < nk; ++it) iterw(std::integral_constant<bool, true>{}, it);
+      for (; it < nk; ++it) iterw(std::integral_constant<bool, false>{}, it);
+    } else {
+      for (; it + C::NST - 1 < nk; ++it) iter(std::integral_constant<bool, true>{}, it);
+      for (; it < nk; ++it) iter(std::integral_constant<bool, false>{}, it);
+    }
   }
 
   // ---- epilogue through LDS.  The accumulators of a 32x32 tile sit column-wise across lanes (lane:
@@ -1047,7 +1125,10 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(GemmArgs g, int spli
 int choose_cfg(const GemmArgs& g) {
   const bool silu = g.epi == Epi::DQ_SILU || g.epi == Epi::DQ_SILU_F32A || g.epi == Epi::SILU_BF16;
   // 5 and 8 (96- and 160-column waves) cannot hold whole [gate | up] blocks
-  auto ok = [&](int id) { return id >= 1 && id <= 8 && !(silu && (id == 5 || id == 8)); };
+  // fp8 stages are one wide k-step, held in four operand sets: with the 256x320 tile's 160 accumulators
+  // they exceed a wave's 256 registers
+  const bool wide320 = !silu && g.in != GemmIn::F8;
+  auto ok = [&](int id) { return id >= 1 && id <= 8 && !(silu && id == 5) && !(!wide320 && id == 8); };
   if (ok(g.cfg)) return g.cfg;
   static const int forced = [] {
     const char* e = std::getenv("MK_GEMM_CFG");   // tuning override: 1 .. 8
@@ -1071,7 +1152,7 @@ int choose_cfg(const GemmArgs& g) {
   int best = 2;
   double bt = 1e300;
   for (const Opt& o : opts) {
-    if (silu && (o.id == 3 || o.id == 5 || o.id == 8)) continue;   // 3: never faster; 5, 8: no SiLU
+    if ((silu && (o.id == 3 || o.id == 5)) || (!wide320 && o.id == 8)) continue;   // 3: never faster; 5, 8: no SiLU
     const double tiles = (double)((g.M + o.bm - 1) / o.bm) * ((g.N + o.bn - 1) / o.bn);
     const double t = std::ceil(tiles / 256.0) * o.bm * o.bn / o.eff;
     if (t < bt * 0.999) {
@@ -1133,7 +1214,7 @@ void launch_t(const GemmArgs& g, hipStream_t st) {
       else launch_c<CfgM, IN, EPI>(g, st);
       break;
     case 8:   // 160-column waves: likewise
-      if constexpr (!silu) launch_c<CfgW, IN, EPI>(g, st);
+      if constexpr (!silu && IN != GemmIn::F8) launch_c<CfgW, IN, EPI>(g, st);
       else launch_c<CfgM, IN, EPI>(g, st);
       break;
     case 6: launch_c<CfgD, IN, EPI>(g, st); break;

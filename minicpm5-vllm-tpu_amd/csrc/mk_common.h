@@ -96,6 +96,16 @@ __device__ inline f32x16 mfma_fp8_32x32x32(const u32x4& a, const u32x4& b, const
   return __builtin_amdgcn_mfma_f32_32x32x16_fp8_fp8(a2[1], b2[1], t, 0, 0, 0);
 }
 
+// The same product over 32 bytes of K per lane (a0, b0 then a1, b1) in one v_mfma_f32_32x32x64_f8f6f4,
+// unscaled, both operands e4m3 (format 0): twice the rate of the K = 16 form above.
+typedef int i32x8 __attribute__((ext_vector_type(8)));
+__device__ inline f32x16 mfma_fp8_32x32x64(const u32x4& a0, const u32x4& a1, const u32x4& b0, const u32x4& b1,
+                                           const f32x16& c) {
+  const i32x8 a = __builtin_shufflevector(bitcast<i32x4>(a0), bitcast<i32x4>(a1), 0, 1, 2, 3, 4, 5, 6, 7);
+  const i32x8 b = __builtin_shufflevector(bitcast<i32x4>(b0), bitcast<i32x4>(b1), 0, 1, 2, 3, 4, 5, 6, 7);
+  return __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(a, b, c, 0, 0, 0, 0, 0, 0);
+}
+
 // f32 -> OCP e4m3 (float8_e4m3fn) with round-to-nearest-even (v_cvt_pk_fp8_f32).  Callers clip to
 // [-448, 448] first, as the reference does before its cast, so no value saturates.
 __device__ inline uint32_t pack_fp8x4(float a, float b, float c, float d) {

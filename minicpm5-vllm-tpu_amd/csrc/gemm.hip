@@ -31,7 +31,11 @@ namespace mk {
 
 namespace {
 
-constexpr int BKB = 64;   // K bytes per LDS stage (two MFMA k-steps)
+// K bytes per LDS stage: 64 (two MFMA k-steps); 128 (four, whole cache lines) in the short-problem loop
+constexpr int stage_kb(int loop) { return loop == 3 ? 128 : 64; }
+// threads per workgroup: the short-problem loop has as many loader waves (they only issue the async loads)
+// as compute waves
+constexpr int block_threads(int wgm, int wgn, int loop) { return 64 * wgm * wgn * (loop == 3 ? 2 : 1); }
 
 // 32-column accumulator tiles per epilogue staging chunk: all NTL of them when the waves' 32-row slices
 // fit in the ring, else the most that do (whole epilogue passes of ew columns each).
@@ -46,27 +50,33 @@ template <int BM_, int BN_, int WGM_, int WGN_, int NST_, int OCC_, int LOOP_ = 
 struct GemmCfg {
   static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, NST = NST_, OCC = OCC_;
   // main loop: 0 split k-step pipeline, 1 ping-pong (two wave groups, operand prefetch), 2 two stages
-  // per barrier with the operands read half a stage ahead
+  // per barrier with the operands read half a stage ahead, 3 128-byte stages with the operands read a whole
+  // stage ahead
   static constexpr int LOOP = LOOP_;
-  static constexpr int NW = WGM * WGN, NTH = 64 * NW;
+  static constexpr int NW = WGM * WGN;                    // compute waves
+  static constexpr int LW = LOOP == 3 ? NW : 0;           // loader waves
+  static constexpr int NTH = block_threads(WGM, WGN, LOOP);
   static constexpr int WM = BM / WGM, WN = BN / WGN;     // wave tile
   static constexpr int MT = WM / 32, NTL = WN / 32;       // 32x32 MFMA tiles per wave
+  static constexpr int BKB = stage_kb(LOOP);
   static constexpr int A_BYTES = BM * BKB, ST_BYTES = (BM + BN) * BKB;
-  // a stage is NL blocks of 16 rows x 64 bytes (1 KB, one async-load instruction): A blocks 0 .. NA-1,
+  // a stage is NL blocks of RPB rows x BKB bytes (1 KB, one async-load instruction): A blocks 0 .. NA-1,
   // then B blocks; block b is loaded by wave b % NW.  Waves w < NL % NW load QH blocks, the rest QL.
-  static constexpr int NA = BM / 16, NL = (BM + BN) / 16;
+  static constexpr int RPB = 1024 / BKB, CPR = BKB / 16;   // rows per block, 16-byte chunks per row
+  static constexpr int NA = BM / RPB, NL = (BM + BN) / RPB;
   static constexpr int QL = NL / NW, QH = (NL + NW - 1) / NW, NQH = NL % NW == 0 ? NW : NL % NW;
   static constexpr int EW = WN % 64 == 0 ? 64 : 32;       // epilogue pass width (columns)
   static constexpr int ECH = epi_chunk(NTL, EW, NW, NST * ST_BYTES);   // 32-column tiles per staging chunk
   static constexpr int NECH = (NTL + ECH - 1) / ECH;
   static constexpr int EROW = ECH * 32 * 4 + 16;          // epilogue LDS row (f32 + pad)
-  static_assert(BM % 16 == 0 && BN % 16 == 0 && NA % NW == 0, "load split: A blocks evenly over the waves");
+  static_assert(BM % RPB == 0 && BN % RPB == 0 && NA % NW == 0, "load split: A blocks evenly over the waves");
   static_assert(LOOP == 1 || NL % NW == 0, "split k-step loop: the same load count on every wave");
   static_assert(NW * 32 * EROW <= NST * ST_BYTES, "epilogue staging fits in the ring");
   static_assert(WN % 32 == 0, "wave tile width");
   // ping-pong: waves w and w + 4 share a SIMD and belong to groups 0 and 1; each group loads a uniform
   // number of blocks per stage
   static_assert(LOOP != 2 || NST >= 5, "two-stage loop: stages it + 2, it + 3 land while it + 4 .. are in flight");
+  static_assert(LOOP != 3 || (NL % NW == 0 && NST >= 3), "whole-stage loop: uniform loads, two stages in flight");
   static_assert(LOOP != 1 || (NW == 8 && NST >= 3 && NQH % 4 == 0),
                 "ping-pong needs two groups of four waves with uniform loads and two stages in flight");
   // Lean addressing for ping-pong tiles whose accumulators and three operand sets nearly fill the 256
@@ -89,10 +99,19 @@ using CfgN = GemmCfg<256, 192, 4, 2, 4, 1, 1>;
 // of 256 CUs at M = 8192 where 256x192 tiles take 1.75 rounds; its epilogue stages 128 + 32 columns
 using CfgW = GemmCfg<256, 320, 4, 2, 4, 1, 1>;
 // Short problems (few tiles, each K loop latency-bound): 8-stage rings, seven stages of loads in flight.
-// 128x128 block, 64x64 per wave; 64x128 block, 32x64 per wave; one workgroup per CU
-// (the 64x128 tile runs two stages per barrier: its waves have few MFMAs per stage to cover a barrier)
-using CfgD = GemmCfg<128, 128, 2, 2, 8, 1>;
+// 64x128 block, 32x64 per wave, one workgroup per CU (the 64x128 tile runs two stages per barrier: its waves
+// have few MFMAs per stage to cover a barrier)
 using CfgE = GemmCfg<64, 128, 2, 2, 8, 1, 2>;
+// Short problems on whole cache lines (128-byte stages, loader waves): 128x128, 64x128, 64x64 (two workgroups
+// per CU) and 32x64 blocks.  What bounds them is the load path of a CU, 64 B/clk at best and 29 - 40 B/clk
+// here, so the smallest tile whose tiling still fits one round of CUs wins: it spreads the same K loop over
+// the most CUs.  Against 64-byte stages, a line's second half no longer comes from L2 a second time, and
+// twice the bytes are in flight when the weights are cold (1B down at M = 256, us warm / cold: 64x128 with
+// 64-byte stages 29.1 / 45.6, this 64x128 24.4 / 33.6, 64x64 17.8 / 23.2, 32x64 17.8 / 19.3).
+using CfgD = GemmCfg<128, 128, 2, 2, 5, 1, 3>;
+using CfgF = GemmCfg<64, 64, 2, 2, 5, 2, 3>;
+using CfgG = GemmCfg<32, 64, 1, 2, 10, 1, 3>;
+using CfgH = GemmCfg<64, 128, 2, 2, 6, 1, 3>;
 
 template <GemmIn IN>
 struct Mma;
@@ -162,10 +181,11 @@ __device__ inline void epi_store(const GemmArgs& g, int m, int n, float v) {
   }
 }
 
-// Stage s of the LDS ring holds A rows [0, BM) then B rows [0, BN), 64 bytes of K each.  16-byte
+// Stage s of the LDS ring holds A rows [0, BM) then B rows [0, BN), BKB bytes of K each.  16-byte
 // chunk c of row r sits at slot c ^ swz(r), so the 16 lanes of a ds_read_b128 phase (16 consecutive
 // rows, same chunk) hit 16 distinct 4-bank groups.
-__device__ inline int swz(int row) { return (row >> 2) & 3; }
+template <int BKB>
+__device__ inline int swz(int row) { return BKB == 64 ? (row >> 2) & 3 : (row >> 1) & 7; }
 
 // Workgroup barrier for the LDS ring.  A bare s_barrier: __syncthreads() adds a fence that would also
 // drain the younger stages' async loads.  The empty asm statements keep the compiler from moving LDS
@@ -181,10 +201,11 @@ __device__ inline void lds_barrier() {
 #define MK_WAIT_VMCNT(n) __builtin_amdgcn_s_waitcnt(((n) & 15) | (7 << 4) | (15 << 8) | (((n) >> 4) << 14))
 
 template <int BM, int BN, int WGM, int WGN, int NST, int OCC, int LOOP, GemmIn IN, Epi EPI>
-__global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kernel(GemmArgs g) {
+__global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kernel(GemmArgs g) {
   using C = GemmCfg<BM, BN, WGM, WGN, NST, OCC, LOOP>;
   using T = Mma<IN>;
   using Acc = typename T::Acc;
+  constexpr int BKB = C::BKB;
   __shared__ __attribute__((aligned(1024))) char smem[C::NST * C::ST_BYTES];
 
   const int tid = threadIdx.x, lane = tid & 63;
@@ -193,7 +214,9 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kernel(GemmArgs g) {
   // QKV routing: the attention's work queues start empty (vector atomics: no scalar-cache writes)
   if (ROUTE && g.queue && blockIdx.x == 0 && blockIdx.y == 0 && tid <= g.n_kv) atomicExch(&g.queue[tid], 0);
   const int col = lane & 31, half = lane >> 5;
-  const int wm = w / C::WGN, wn = w % C::WGN;
+  const bool loader = C::LW > 0 && w >= C::NW;
+  const int lw = loader ? w - C::NW : w;                   // block set of the async loads (C::LW > 0: loaders only)
+  const int wm = lw / C::WGN, wn = lw % C::WGN;
   // Tile order.  Workgroups are dispatched round-robin over the 8 XCDs, each with its own L2: launch id
   // lid runs on XCD lid % 8, so XCD x is given the contiguous work range [x, x + 1) * nblk / 8.  Work
   // ids walk GM-row groups column by column, so the ~32-64 tiles an XCD runs at once form a compact
@@ -211,20 +234,20 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kernel(GemmArgs g) {
   constexpr int Q = C::QH;
   const bool qfull = C::QH == C::QL || w < C::NQH;
 
-  // this lane's async-load sources: block b = w + NW j, rows 16 (b or b - NA) + lane / 4 of A or B, as
+  // this lane's async-load sources: block b = w + NW j, rows RPB (b or b - NA) + lane / CPR of A or B, as
   // 32-bit byte offsets from the operand base (the base and the K offset stay scalar); rows past M / N
   // are clamped (their results are never stored)
   constexpr int JA = C::NA / C::NW;                       // load instructions j < JA are A blocks
   uint32_t loff[Q];
 #pragma unroll
   for (int j = 0; j < Q; ++j) {
-    const int b = w + C::NW * j;
+    const int b = lw + C::NW * j;
     if (j < JA) {
-      const int r = 16 * b + (lane >> 2);
-      loff[j] = (uint32_t)min(m0 + r, g.M - 1) * (uint32_t)lda + 16u * ((lane & 3) ^ swz(r));
+      const int r = C::RPB * b + lane / C::CPR;
+      loff[j] = (uint32_t)min(m0 + r, g.M - 1) * (uint32_t)lda + 16u * ((lane % C::CPR) ^ swz<BKB>(r));
     } else {
-      const int r = 16 * (b - C::NA) + (lane >> 2);
-      loff[j] = (uint32_t)min(n0 + r, g.N - 1) * (uint32_t)ldb + 16u * ((lane & 3) ^ swz(r));
+      const int r = C::RPB * (b - C::NA) + lane / C::CPR;
+      loff[j] = (uint32_t)min(n0 + r, g.N - 1) * (uint32_t)ldb + 16u * ((lane % C::CPR) ^ swz<BKB>(r));
     }
   }
   // Lean addressing: load j's rows are 16 NW j rows past load 0's (A) or load JA's (B), with the same
@@ -232,7 +255,8 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kernel(GemmArgs g) {
   // 16-byte chunk plus the largest K offset still ends inside the buffer (the range check covers the
   // lane offset only).  The empty asm keeps the sum from being hoisted out of the loop into a register
   // of its own.
-  const uint32_t lim_a = (uint32_t)(g.M - 1) * (uint32_t)lda + 48u, lim_b = (uint32_t)(g.N - 1) * (uint32_t)ldb + 48u;
+  const uint32_t lim_a = (uint32_t)(g.M - 1) * (uint32_t)lda + 16u * (C::CPR - 1),
+                 lim_b = (uint32_t)(g.N - 1) * (uint32_t)ldb + 16u * (C::CPR - 1);
   constexpr bool LEAN = C::LEAN || (T::WIDE && C::LOOP == 1 && 16 * C::MT * C::NTL + 16 * (C::MT + C::NTL) > 216);
   auto voff = [&](int j) -> uint32_t {
     if constexpr (!LEAN) {
@@ -242,7 +266,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kernel(GemmArgs g) {
       if (j == 0 || j == JA) return loff[j];
       uint32_t o = isa ? loff[0] : loff[JA];
       asm volatile("" : "+v"(o));
-      o += (uint32_t)((isa ? j : j - JA) * 16 * C::NW) * (uint32_t)(isa ? lda : ldb);
+      o += (uint32_t)((isa ? j : j - JA) * C::RPB * C::NW) * (uint32_t)(isa ? lda : ldb);
       return min(o, isa ? lim_a : lim_b);
     }
   };
@@ -255,7 +279,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kernel(GemmArgs g) {
   // async load j (of Q) of stage `st` at K byte offset kb; block b sits at b KB in the stage (A blocks,
   // then B blocks)
   auto issue1 = [&](int j, int st, int kb) {
-    char* dst = smem + st * C::ST_BYTES + (w + C::NW * j) * 1024;
+    char* dst = smem + st * C::ST_BYTES + (lw + C::NW * j) * 1024;
     if (j < JA) copy16_to_lds(rA, voff(j), (uint32_t)kb, dst);
     else if (j < C::QL || qfull) copy16_to_lds(rB, voff(j), (uint32_t)kb, dst);
   };
@@ -267,6 +291,16 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kernel(GemmArgs g) {
     else MK_WAIT_VMCNT(n * C::QL);
   };
   using W0 = std::integral_constant<int, 0>;
+  // wait until at most min(n, left) stages are outstanding (left: stages there are beyond the one waited for)
+  auto wait_newer = [&](auto nc, int left) {
+    auto go = [&](auto self, auto c) -> void {
+      constexpr int n = decltype(c)::value;
+      if constexpr (n <= 0) wait_stages(W0{});
+      else if (left >= n) wait_stages(c);
+      else self(self, std::integral_constant<int, n - 1>{});
+    };
+    go(go, nc);
+  };
 
   Acc acc[C::MT][C::NTL];
 #pragma unroll
@@ -276,7 +310,7 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kernel(GemmArgs g) {
 
   // LDS operand reads.  Row wm WM + 32 mt + col of A has swizzle swz(col) (WM and 32 are multiples of
   // 16), so tile mt is a fixed 2 KB step from tile 0 and the per-k-step lane offsets are two registers.
-  const int sw = swz(col);
+  const int sw = swz<BKB>(col);
   const int aro = (wm * C::WM + col) * BKB, bro = C::A_BYTES + (wn * C::WN + col) * BKB;
   const int ao0 = aro + 16 * (half ^ sw), ao1 = aro + 16 * ((2 + half) ^ sw);
   const int bo0 = bro + 16 * (half ^ sw), bo1 = bro + 16 * ((2 + half) ^ sw);
@@ -349,20 +383,24 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kernel(GemmArgs g) {
   };
   // the scales are held through the main loop only when they take few registers
   constexpr bool EARLY_SCALES = C::MT * NTASK + NSB * (SILU ? 16 : 8) <= 32;
-  if (EARLY_SCALES && dq) load_scales();
+  if (EARLY_SCALES && dq && !loader) load_scales();
 
-  const int nk = Kb / BKB;
+  const int nk = Kb / BKB;   // stages
   // stages loaded ahead of the main loop: NST - 1 (NST - 2 for the two-stage loop, whose iterations
-  // load two stages each); stage 0 (stages 0 and 1) visible after the barrier
-  constexpr int PRE = C::LOOP == 2 ? C::NST - 2 : C::NST - 1;
+  // load two stages each; stages 0 and 1 visible after the barrier there, stage 0 in the others)
+  // (every slot for the whole-stage loop); stages 0 and 1 visible after the barrier
+  constexpr int PRE = C::LOOP == 3 ? C::NST : C::LOOP == 2 ? C::NST - 2 : C::NST - 1;
+  if (C::LW == 0 || loader) {
 #pragma unroll
-  for (int s0 = 0; s0 < PRE; ++s0)
-    if (s0 < nk) {
+    for (int s0 = 0; s0 < PRE; ++s0)
+      if (s0 < nk) {
 #pragma unroll
-      for (int j = 0; j < Q; ++j) issue1(j, s0, s0 * BKB);
-    }
-  if (nk >= PRE) wait_stages(std::integral_constant<int, C::LOOP == 2 ? PRE - 2 : PRE - 1>{});
-  else wait_stages(W0{});
+        for (int j = 0; j < Q; ++j) issue1(j, s0, s0 * BKB);
+      }
+    if (C::LOOP == 3) wait_newer(std::integral_constant<int, PRE - 2>{}, nk - 2);
+    else if (nk >= PRE) wait_stages(std::integral_constant<int, C::LOOP >= 2 ? PRE - 2 : PRE - 1>{});
+    else wait_stages(W0{});
+  }
   lds_barrier();
   // Materialize the epilogue's kernel arguments now: a scalar load still pending inside the loop would
   // turn every LDS wait there into lgkmcnt(0) (scalar loads return out of order).
@@ -571,6 +609,69 @@ __global__ __launch_bounds__(64 * WGM * WGN, OCC) void gemm_kernel(GemmArgs g) {
     int it = 0;
     for (; it + C::NST - 1 < nk; it += 2) iter2(std::integral_constant<bool, true>{}, it);
     for (; it < nk; it += 2) iter2(std::integral_constant<bool, false>{}, it);
+  } else if constexpr (C::LOOP == 3) {
+    // One 128-byte stage (k-steps 0 .. 3) per iteration and barrier.  The loader waves issue the async loads,
+    // the compute waves read LDS and issue MFMAs: in one wave the three queue behind each other (in-order
+    // issue), ~460 cycles per stage of a 32x64 tile whose loads alone take 192 at 64 B/clk.  A compute wave
+    // has a stage's operands in registers since the iteration before, so the reads of stage it + 1 run under
+    // the MFMAs of stage it.  Stage it's slot was read in iteration it - 1 (lgkmcnt(0) ahead of its barrier),
+    // so the loads of stage it + NST go there.  Both kinds of waves meet at one barrier per iteration.
+    // The MFMAs of an output element run over the k-steps in the same order as in the other loops.
+    if (loader) {
+      lds_barrier();   // the compute waves have read stage 0
+      int cur = 0;     // slot of stage it
+      for (int it = 0; it + 1 < nk; ++it) {
+        if (it + C::NST < nk) {
+#pragma unroll
+          for (int j = 0; j < Q; ++j) issue1(j, cur, (it + C::NST) * BKB);
+          wait_stages(std::integral_constant<int, C::NST - 2>{});
+        } else {
+          wait_newer(std::integral_constant<int, C::NST - 3>{}, nk - 3 - it);
+        }
+        lds_barrier();   // stage it + 2 landed
+        cur = cur == C::NST - 1 ? 0 : cur + 1;
+      }
+      lds_barrier();   // the epilogue's: every compute wave is done with the ring
+      return;
+    }
+    u32x4 ya[2][4][C::MT], yb[2][4][C::NTL];
+    auto rd4 = [&](const char* S, u32x4 (&ra)[4][C::MT], u32x4 (&rb)[4][C::NTL]) {
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        const int x = 16 * ((2 * ks + half) ^ sw);
+#pragma unroll
+        for (int nt = 0; nt < C::NTL; ++nt) rb[ks][nt] = *reinterpret_cast<const u32x4*>(S + bro + x + nt * 32 * BKB);
+#pragma unroll
+        for (int mt = 0; mt < C::MT; ++mt) ra[ks][mt] = *reinterpret_cast<const u32x4*>(S + aro + x + mt * 32 * BKB);
+      }
+    };
+    rd4(smem, ya[0], yb[0]);
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    lds_barrier();
+    int cur = 0;   // slot of stage it
+    auto iter3 = [&](int it, auto set) {
+      constexpr int X = decltype(set)::value;
+      const bool more = it + 1 < nk;
+      cur = cur == C::NST - 1 ? 0 : cur + 1;
+      if (more) rd4(smem + cur * C::ST_BYTES, ya[X ^ 1], yb[X ^ 1]);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int ks = 0; ks < 4; ks += T::WIDE ? 2 : 1)
+#pragma unroll
+        for (int i = 0; i < NMF; ++i) {
+          if constexpr (T::WIDE) mfw(i, ya[X][ks], yb[X][ks], ya[X][ks + 1], yb[X][ks + 1]);
+          else mf(i, ya[X][ks], yb[X][ks]);
+        }
+      __builtin_amdgcn_sched_barrier(0);
+      if (more) {
+        __builtin_amdgcn_s_waitcnt(0xc07f);   // this wave's reads of stage it + 1 are done
+        lds_barrier();
+      }
+    };
+    for (int it = 0; it < nk; it += 2) {
+      iter3(it, std::integral_constant<int, 0>{});
+      if (it + 1 < nk) iter3(it + 1, std::integral_constant<int, 1>{});
+    }
   } else {
     u32x4 ra0[C::MT], rb0[C::NTL], ra1[C::MT], rb1[C::NTL];
     rd(smem, ao0, bo0, ra0, rb0);
@@ -1128,23 +1229,42 @@ int choose_cfg(const GemmArgs& g) {
   // fp8 stages are one wide k-step, held in four operand sets: with the 256x320 tile's 160 accumulators
   // they exceed a wave's 256 registers
   const bool wide320 = !silu && g.in != GemmIn::F8;
-  auto ok = [&](int id) { return id >= 1 && id <= 8 && !(silu && id == 5) && !(!wide320 && id == 8); };
+  const int kb = g.K * (g.in == GemmIn::BF16 ? 2 : 1);   // bytes
+  const bool line = kb % 128 == 0;                        // whole 128-byte stages
+  // 5, 8, 9, 10: waves without whole [gate | up] blocks; 6, 9 - 12: 128-byte stages
+  auto ok = [&](int id) {
+    if (id == 8) return wide320;
+    if (silu) return id >= 1 && id <= 7 && id != 5 && id != 6;
+    return id >= 1 && id <= 11 && (line || !(id == 6 || id >= 9));
+  };
   if (ok(g.cfg)) return g.cfg;
   static const int forced = [] {
     const char* e = std::getenv("MK_GEMM_CFG");   // tuning override: 1 .. 8
     return e ? std::atoi(e) : 0;
   }();
   if (ok(forced)) return forced;
-  // Few tiles (short prompts, e.g. M <= 1024): each tile's K loop is latency-bound, so the 64x128 tile
-  // whose loop runs two stages per barrier wins whenever its tiling fits one round of 256 CUs (measured
-  // on MI355X at M = 128 - 1024: the 1B gate/up at M = 128 takes 7.6 us on it, 14.0 on 256x128; the 1B
-  // down at M = 1024 31.9 us, 40.3 on the 128x128 deep ring, 48.4 on the 128x128 three-workgroup
-  // tile); otherwise the 128x128 deep ring for long K loops, else the wide tiles.
+  // Few tiles (short prompts): the smallest tile whose tiling fits one round of 256 CUs, on whole-line stages.
+  // Measured on MI355X over M = 40 .. 3072 at the model's shapes, us warm / with cold weights, against the next
+  // larger choice:
+  //   32x64   1B down M = 256  17.8 / 19.3 (64x64 17.8 / 23.2), 2B down M = 128  21.9 / 25.0 (22.1 / 31.3)
+  //   64x64   1B down M = 512  19.1 / 23.4 (64x128 25.4 / 33.5), 1B QKV M = 384  6.5 / 7.1 (8.1 / 9.7)
+  //   64x128  1B down M = 1024  27.3 / 32.9 (64x128 with 64-byte stages 30.5 / 43.6); K loops of 32 or more
+  //           lines only: at 12 (int8, K = 1536) the 64-byte stages start sooner, 7.5 against 8.3 at M = 512
+  //   128x128 1B down M = 2048  40.4 / 43.6 (64-byte stages 44.3 / 55.0), likewise for 32 or more lines
+  // The SiLU epilogues need 64-column waves: 64x128 with 64-byte stages (1B gate/up M = 128  6.9 / 11.8 against
+  // 7.9 / 9.9 on whole lines), then 128x128 with three workgroups per CU (M = 256  9.6 / 14.2 against
+  // 13.7 / 17.8 on 256x128 tiles, M = 384  11.0 / 14.6 against 14.8 / 17.9).
   {
-    const int nk = g.K * (g.in == GemmIn::BF16 ? 2 : 1) / BKB;
-    auto tiles = [&](int bm, int bn) { return (long)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn); };
-    if (nk >= 16 && tiles(64, 128) <= 256) return 7;
-    if (nk >= 64 && tiles(128, 128) <= 256) return 6;
+    const int lines = kb / 128;
+    auto fits = [&](int bm, int bn) { return (long)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn) <= 256; };
+    if (!silu && line) {
+      if (fits(32, 64)) return 10;
+      if (fits(64, 64)) return 9;
+      if (lines >= 32 && fits(64, 128)) return 11;
+    }
+    if (kb >= 1024 && fits(64, 128)) return 7;
+    if (!silu && line && lines >= 32 && fits(128, 128)) return 6;
+    if (silu && fits(128, 128)) return 3;
   }
   struct Opt { int id, bm, bn; double eff; };
   const Opt opts[6] = {{4, 256, 256, silu ? 1.05 : 1.25}, {2, 256, 128, 1.0}, {1, 256, 256, 0.9},
@@ -1217,8 +1337,19 @@ void launch_t(const GemmArgs& g, hipStream_t st) {
       if constexpr (!silu && IN != GemmIn::F8) launch_c<CfgW, IN, EPI>(g, st);
       else launch_c<CfgM, IN, EPI>(g, st);
       break;
-    case 6: launch_c<CfgD, IN, EPI>(g, st); break;
+    case 6:
+      if constexpr (!silu) launch_c<CfgD, IN, EPI>(g, st);
+      break;
     case 7: launch_c<CfgE, IN, EPI>(g, st); break;
+    case 9:
+      if constexpr (!silu) launch_c<CfgF, IN, EPI>(g, st);
+      break;
+    case 10:
+      if constexpr (!silu) launch_c<CfgG, IN, EPI>(g, st);
+      break;
+    case 11:
+      if constexpr (!silu) launch_c<CfgH, IN, EPI>(g, st);
+      break;
     default: launch_c<CfgM, IN, EPI>(g, st); break;
   }
 }
@@ -1346,7 +1477,7 @@ int gemm_validate(const GemmArgs& g) {
 int launch_gemm(const GemmArgs& g, hipStream_t st) {
   int rc = gemm_validate(g);
   if (rc) return rc;
-  MK_REQUIRE((g.K * (g.in == GemmIn::BF16 ? 2 : 1)) % BKB == 0, "gemm: K bytes must be a multiple of 64");
+  MK_REQUIRE((g.K * (g.in == GemmIn::BF16 ? 2 : 1)) % 64 == 0, "gemm: K bytes must be a multiple of 64");
   MK_REQUIRE(g.N % 8 == 0 && (g.ldo % 8 == 0) && (g.ldr % 8 == 0), "gemm: N and output strides must be multiples of 8");
   {
     const uint64_t esz = g.in == GemmIn::BF16 ? 2 : 1;

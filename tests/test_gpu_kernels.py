@@ -267,6 +267,31 @@ def test_gemm_bf16_rows_independent_of_tile(N, K):
     assert torch.equal(small.view(torch.int32), big[:1000].view(torch.int32))
 
 
+@pytest.mark.parametrize("M,N,K", [(33, 72, 64), (40, 1536, 192), (250, 1504, 4608), (321, 1528, 128), (500, 1504, 320),
+                                   (1000, 1512, 2112), (600, 1512, 2048), (2000, 1512, 2112), (1100, 1512, 2048)])
+def test_gemm_short_problem_tiles(M, N, K):
+    """Whole-line tiles of short problems (32x64, 64x64, 64x128, 128x128: K loops of one stage, fewer stages
+    than ring slots, an odd and an even count; ragged rows and columns): bf16 rows bitwise equal to the same rows of a
+    product of 9000 rows on a wide tile and within 64 eps sum|products| of float64; int8 exact."""
+    from minicpm5_mk import ops
+
+    dev = _dev()
+    g = torch.Generator().manual_seed(M + N + K)
+    print(f"[short tiles] {M}x{N}x{K}", flush=True)
+    a = torch.randn(9000, K, generator=g).to(BF16).to(dev)
+    b = (torch.randn(N, K, generator=g) * 0.02).to(BF16).to(dev)
+    out, big = ops.gemm(a[:M].contiguous(), b, "f32"), ops.gemm(a, b, "f32")
+    assert torch.equal(out.view(torch.int32), big[:M].view(torch.int32))
+    ref = a[:M].double() @ b.double().t()
+    assert ((out.double() - ref).abs() <= 64 * 2.0 ** -24 * (a[:M].double().abs() @ b.double().abs().t())).all()
+    x = torch.randn(M, N, generator=g).to(BF16).to(dev)
+    res = ops.gemm(a[:M].contiguous(), b, "res_f32add", res=x.clone())
+    assert torch.equal(res.view(torch.int16), (x.float() + out).to(BF16).view(torch.int16))
+    ai = torch.randint(-127, 128, (M, 2 * K), generator=g, dtype=torch.int8).to(dev)
+    bi = torch.randint(-127, 128, (N, 2 * K), generator=g, dtype=torch.int8).to(dev)
+    assert torch.equal(ops.gemm(ai, bi, "i32").double(), ai.double() @ bi.double().t())
+
+
 @pytest.mark.parametrize("epi", ["f32", "bf16", "res_f32add", "res_bf16add"])
 def test_gemm_wide_tile_rows_match(epi):
     """M = 8192, N = 2560 takes the 256x320 tile (one round of 256 CUs; 64x160 wave tiles, the epilogue

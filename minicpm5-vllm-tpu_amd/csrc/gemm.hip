@@ -32,7 +32,7 @@ namespace mk {
 namespace {
 
 // K bytes per LDS stage: 64 (two MFMA k-steps); 128 (four, whole cache lines) in the short-problem loop
-constexpr int stage_kb(int loop) { return loop == 3 ? 128 : 64; }
+constexpr int stage_kb(int loop) { return loop >= 3 ? 128 : 64; }
 // threads per workgroup: the short-problem loop has as many loader waves (they only issue the async loads)
 // as compute waves
 constexpr int block_threads(int wgm, int wgn, int loop) { return 64 * wgm * wgn * (loop == 3 ? 2 : 1); }
@@ -51,7 +51,7 @@ struct GemmCfg {
   static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, NST = NST_, OCC = OCC_;
   // main loop: 0 split k-step pipeline, 1 ping-pong (two wave groups, operand prefetch), 2 two stages
   // per barrier with the operands read half a stage ahead, 3 128-byte stages with the operands read a whole
-  // stage ahead
+  // stage ahead and loader waves, 4 ping-pong over 128-byte stages in two slots
   static constexpr int LOOP = LOOP_;
   static constexpr int NW = WGM * WGN;                    // compute waves
   static constexpr int LW = LOOP == 3 ? NW : 0;           // loader waves
@@ -70,6 +70,7 @@ struct GemmCfg {
   static constexpr int NECH = (NTL + ECH - 1) / ECH;
   static constexpr int EROW = ECH * 32 * 4 + 16;          // epilogue LDS row (f32 + pad)
   static_assert(BM % RPB == 0 && BN % RPB == 0 && NA % NW == 0, "load split: A blocks evenly over the waves");
+  static_assert(LOOP != 4 || (NW == 8 && NST == 2 && NL % NW == 0), "two-slot ping-pong: two groups of four waves");
   static_assert(LOOP == 1 || NL % NW == 0, "split k-step loop: the same load count on every wave");
   static_assert(NW * 32 * EROW <= NST * ST_BYTES, "epilogue staging fits in the ring");
   static_assert(WN % 32 == 0, "wave tile width");
@@ -82,7 +83,7 @@ struct GemmCfg {
   // Lean addressing for ping-pong tiles whose accumulators and three operand sets nearly fill the 256
   // registers of a wave: the async-load lane offsets that follow from others are recomputed where
   // they are used instead of being held through the main loop (held, they spilled into the loop).
-  static constexpr bool LEAN = LOOP == 1 && 16 * MT * NTL + 12 * (MT + NTL) > 232;
+  static constexpr bool LEAN = (LOOP == 1 || LOOP == 4) && 16 * MT * NTL + 12 * (MT + NTL) > (LOOP == 4 ? 190 : 232);
 };
 // 256x256 block, 128x128 per wave (accumulators in AGPRs), one workgroup per CU
 using CfgL = GemmCfg<256, 256, 2, 2, 3, 1, 0>;
@@ -90,11 +91,13 @@ using CfgL = GemmCfg<256, 256, 2, 2, 3, 1, 0>;
 using CfgM = GemmCfg<256, 128, 2, 2, 3, 2>;
 // 128x128 block, 64x64 per wave, three workgroups per CU
 using CfgS = GemmCfg<128, 128, 2, 2, 3, 3>;
-// 256x256 block, 8 waves of 128x64 (two per SIMD), one workgroup per CU
-using CfgX = GemmCfg<256, 256, 2, 4, 4, 1, 1>;
+// 256x256 block, 8 waves of 128x64 (two per SIMD), one workgroup per CU, 128-byte stages (whole cache lines;
+// us at M = 8192 against 64-byte stages in a four-slot ring: 2B down 171 -> 161, 2B gate/up 201 -> 188, and the
+// 1B gate/up 125 against 130 on pairs of 256x128 tiles; 256x192: 1B down 106 -> 96, O 53.1 -> 48.9)
+using CfgX = GemmCfg<256, 256, 2, 4, 2, 1, 4>;
 // 256x192 block, 8 waves of 64x96 (two per SIMD), one workgroup per CU: N = 1536 in 8 column tiles, so
 // M = 8192 fills exactly 256 CUs
-using CfgN = GemmCfg<256, 192, 4, 2, 4, 1, 1>;
+using CfgN = GemmCfg<256, 192, 4, 2, 2, 1, 4>;
 // 256x320 block, 8 waves of 64x160: N = 2560 (the QKV projection at hd 128) in 8 column tiles, one round
 // of 256 CUs at M = 8192 where 256x192 tiles take 1.75 rounds; its epilogue stages 128 + 32 columns
 using CfgW = GemmCfg<256, 320, 4, 2, 4, 1, 1>;
@@ -257,7 +260,7 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
   // of its own.
   const uint32_t lim_a = (uint32_t)(g.M - 1) * (uint32_t)lda + 16u * (C::CPR - 1),
                  lim_b = (uint32_t)(g.N - 1) * (uint32_t)ldb + 16u * (C::CPR - 1);
-  constexpr bool LEAN = C::LEAN || (T::WIDE && C::LOOP == 1 && 16 * C::MT * C::NTL + 16 * (C::MT + C::NTL) > 216);
+  constexpr bool LEAN = C::LEAN || (T::WIDE && C::LOOP == 4 && 16 * C::MT * C::NTL + 16 * (C::MT + C::NTL) > 216);
   auto voff = [&](int j) -> uint32_t {
     if constexpr (!LEAN) {
       return loff[j];
@@ -282,6 +285,11 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
     char* dst = smem + st * C::ST_BYTES + (lw + C::NW * j) * 1024;
     if (j < JA) copy16_to_lds(rA, voff(j), (uint32_t)kb, dst);
     else if (j < C::QL || qfull) copy16_to_lds(rB, voff(j), (uint32_t)kb, dst);
+  };
+  // A last stage of half the K bytes (LOOP 4): its other half would read past the row (unused), and past the
+  // last row out of the buffer, so the K offset goes where the range check sees it (out of range: zeros).
+  auto issue_half = [&](int j, int st, int kb) {
+    copy16_to_lds(j < JA ? rA : rB, voff(j) + (uint32_t)kb, smem + st * C::ST_BYTES + (lw + C::NW * j) * 1024);
   };
   // wait until at most `n` stages of this wave's async loads are outstanding
   auto wait_stages = [&](auto nc) {
@@ -385,20 +393,23 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
   constexpr bool EARLY_SCALES = C::MT * NTASK + NSB * (SILU ? 16 : 8) <= 32;
   if (EARLY_SCALES && dq && !loader) load_scales();
 
-  const int nk = Kb / BKB;   // stages
+  const int nk = C::LOOP == 4 ? (Kb + BKB - 1) / BKB : Kb / BKB;   // stages
   // stages loaded ahead of the main loop: NST - 1 (NST - 2 for the two-stage loop, whose iterations
   // load two stages each; stages 0 and 1 visible after the barrier there, stage 0 in the others)
   // (every slot for the whole-stage loop); stages 0 and 1 visible after the barrier
-  constexpr int PRE = C::LOOP == 3 ? C::NST : C::LOOP == 2 ? C::NST - 2 : C::NST - 1;
+  constexpr int PRE = C::LOOP >= 3 ? C::NST : C::LOOP == 2 ? C::NST - 2 : C::NST - 1;
   if (C::LW == 0 || loader) {
 #pragma unroll
     for (int s0 = 0; s0 < PRE; ++s0)
-      if (s0 < nk) {
+      if (C::LOOP == 4 && s0 < nk && (s0 + 1) * BKB > Kb) {
+#pragma unroll
+        for (int j = 0; j < Q; ++j) issue_half(j, s0, s0 * BKB);
+      } else if (s0 < nk) {
 #pragma unroll
         for (int j = 0; j < Q; ++j) issue1(j, s0, s0 * BKB);
       }
     if (C::LOOP == 3) wait_newer(std::integral_constant<int, PRE - 2>{}, nk - 2);
-    else if (nk >= PRE) wait_stages(std::integral_constant<int, C::LOOP >= 2 ? PRE - 2 : PRE - 1>{});
+    else if (nk >= PRE) wait_stages(std::integral_constant<int, C::LOOP == 2 || C::LOOP == 3 ? PRE - 2 : PRE - 1>{});
     else wait_stages(W0{});
   }
   lds_barrier();
@@ -419,7 +430,7 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
     constexpr int D = C::NST - 1;
     constexpr int NOP = C::MT + C::NTL;                   // operand registers per k-step: B then A
     u32x4 H0[NOP], H1[NOP], H2[NOP];
-    u32x4 H3[T::WIDE ? NOP : 1];   // WIDE: stage s uses sets (H0, H1) or (H2, H3), all of a stage at once
+    static_assert(!T::WIDE, "one k-step per operand set");
     auto rdq = [&](const char* Sb, int ks, int q, u32x4 (&dst)[NOP]) {
       if (q < C::NTL) dst[q] = *reinterpret_cast<const u32x4*>(Sb + (ks ? bo1 : bo0) + q * 32 * BKB);
       else dst[q] = *reinterpret_cast<const u32x4*>(Sb + (ks ? ao1 : ao0) + (q - C::NTL) * 32 * BKB);
@@ -427,11 +438,6 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
     auto mfq = [&](int i, const u32x4 (&src)[NOP]) {
       const int mt = i / C::NTL, nt = i % C::NTL;
       acc[mt][nt] = T::run(src[C::NTL + mt], src[nt], acc[mt][nt]);
-    };
-    auto mfqw = [&](int i, const u32x4 (&s0)[NOP], const u32x4 (&s1)[NOP]) {
-      const int mt = i / C::NTL, nt = i % C::NTL;
-      if constexpr (T::WIDE)
-        acc[mt][nt] = mfma_fp8_32x32x64(s0[C::NTL + mt], s1[C::NTL + mt], s0[nt], s1[nt], acc[mt][nt]);
     };
     // stages 0 and 1 visible; stage 0 in H0 / H1
     if (nk >= D) wait_stages(std::integral_constant<int, D - 2>{});
@@ -449,7 +455,7 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
     int cur = 0;
     // `steady` instances (stage it + D exists) have no runtime conditions, so the compute phase stays one
     // basic block instead of a branch around every operand read
-    auto step = [&](auto steady, int it, u32x4 (&ha)[NOP], u32x4 (&hb)[NOP], u32x4 (&hc)[NOP], u32x4 (&hd)[NOP]) {
+    auto step = [&](auto steady, int it, u32x4 (&ha)[NOP], u32x4 (&hb)[NOP], u32x4 (&hc)[NOP]) {
       constexpr bool ST = decltype(steady)::value;
       // M(it): async loads of stage it + D into the slot of stage it - 1
       const bool pre = ST || it + D < nk;
@@ -468,36 +474,24 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
       const char* S1 = smem + s1 * C::ST_BYTES;
       const bool nxt = ST || it + 1 < nk;
       __builtin_amdgcn_s_setprio(1);
-      if constexpr (T::WIDE) {
-        constexpr int NRD = 2 * NOP, RPM = (NRD + NMF - 1) / NMF;   // operand reads per MFMA
 #pragma unroll
-        for (int i = 0; i < NMF; ++i) {
-          mfqw(i, ha, hb);
-#pragma unroll
-          for (int q = i * RPM; q < (i + 1) * RPM && q < NRD; ++q)
-            if (nxt) rdq(S1, q & 1, q >> 1, q & 1 ? hd : hc);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-      } else {
-#pragma unroll
-        for (int i = 0; i < NMF; ++i) {
-          mfq(i, ha);
-          if (i < NOP && nxt) rdq(S1, 0, i, hc);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int q = NMF; q < NOP; ++q)
-          if (nxt) rdq(S1, 0, q, hc);
-#pragma unroll
-        for (int i = 0; i < NMF; ++i) {
-          mfq(i, hb);
-          if (i < NOP && nxt) rdq(S1, 1, i, ha);
-          __builtin_amdgcn_sched_barrier(0);
-        }
-#pragma unroll
-        for (int q = NMF; q < NOP; ++q)
-          if (nxt) rdq(S1, 1, q, ha);
+      for (int i = 0; i < NMF; ++i) {
+        mfq(i, ha);
+        if (i < NOP && nxt) rdq(S1, 0, i, hc);
+        __builtin_amdgcn_sched_barrier(0);
       }
+#pragma unroll
+      for (int q = NMF; q < NOP; ++q)
+        if (nxt) rdq(S1, 0, q, hc);
+#pragma unroll
+      for (int i = 0; i < NMF; ++i) {
+        mfq(i, hb);
+        if (i < NOP && nxt) rdq(S1, 1, i, ha);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int q = NMF; q < NOP; ++q)
+        if (nxt) rdq(S1, 1, q, ha);
       __builtin_amdgcn_s_setprio(0);
       __builtin_amdgcn_s_waitcnt(0xc07f);                 // lgkmcnt(0): stage it + 1 is in registers
       if (wgrp == 1 && (ST || it + 2 < nk)) {
@@ -510,26 +504,144 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
     using Steady = std::integral_constant<bool, true>;
     using Tail = std::integral_constant<bool, false>;
     int it = 0;
+    for (; it + 2 + D < nk; it += 3) {
+      step(Steady{}, it, H0, H1, H2);
+      step(Steady{}, it + 1, H2, H0, H1);
+      step(Steady{}, it + 2, H1, H2, H0);
+    }
+    for (; it < nk; it += 3) {
+      step(Tail{}, it, H0, H1, H2);
+      if (it + 1 < nk) step(Tail{}, it + 1, H2, H0, H1);
+      if (it + 2 < nk) step(Tail{}, it + 2, H1, H2, H0);
+    }
+    if (wgrp == 0) lds_barrier();
+  } else if constexpr (C::LOOP == 4) {
+    // Ping-pong over 128-byte stages in two LDS slots: whole cache lines per row, two half-stages (64 bytes of
+    // K) of MFMAs per stage.  With 64-byte slices every load of a line's other half, a stage later, misses
+    // the 32 KB L1 again and L2 delivers each line twice.
+    // Half-stage h = 2 p + (0 or 1) of stage p; phases M(h), C(h) per half-stage as in the loop above, C(h)
+    // reading half-stage h + 1.  Number the barrier intervals so that group 0 runs M(h) in 2h and C(h) in
+    // 2h + 1, group 1 M(h) in 2h + 1 and C(h) in 2h + 2.  Stage p - 1's last reads (half 2p - 1) are in
+    // C(2p - 2): intervals 4p - 3 and 4p - 2, so its slot takes stage p + 1 from interval 4p - 1 on: group 1
+    // loads it in M(2p - 1) (4p - 1), group 0 in M(2p) (4p).  Its first reads are group 0's C(2p + 1), interval
+    // 4p + 3: both groups wait for their loads at the end of 4p + 2 (group 0: M(2p + 1), group 1: C(2p)),
+    // three to four intervals after issuing them.
+    constexpr int NOP = C::MT + C::NTL;                   // operand registers per k-step: B then A
+    u32x4 H0[NOP], H1[NOP], H2[NOP];
+    u32x4 H3[T::WIDE ? NOP : 1];   // WIDE: half-stage h uses sets (H0, H1) or (H2, H3), all of it at once
+    const int nh = Kb / 64;                               // the last stage may hold one half-stage only
+    // operand addresses of the half-stage being read (A and B, k-step 0 and 1): a half is bit 6 of the offset.
+    // They are stepped in place; left to the compiler, every slot and half got a register of its own.
+    int pa0 = ao0, pa1 = ao1, pb0 = bo0, pb1 = bo1;
+    auto advance = [&](int d) {
+      pa0 = (pa0 ^ 64) + d;
+      pa1 = (pa1 ^ 64) + d;
+      pb0 = (pb0 ^ 64) + d;
+      pb1 = (pb1 ^ 64) + d;
+      asm volatile("" : "+v"(pa0), "+v"(pa1), "+v"(pb0), "+v"(pb1));
+    };
+    auto rdq = [&](int ks, int q, u32x4 (&dst)[NOP]) {
+      if (q < C::NTL) dst[q] = *reinterpret_cast<const u32x4*>(smem + (ks ? pb1 : pb0) + q * 32 * BKB);
+      else dst[q] = *reinterpret_cast<const u32x4*>(smem + (ks ? pa1 : pa0) + (q - C::NTL) * 32 * BKB);
+    };
+    auto mfq = [&](int i, const u32x4 (&src)[NOP]) {
+      const int mt = i / C::NTL, nt = i % C::NTL;
+      acc[mt][nt] = T::run(src[C::NTL + mt], src[nt], acc[mt][nt]);
+    };
+    auto mfqw = [&](int i, const u32x4 (&s0)[NOP], const u32x4 (&s1)[NOP]) {
+      const int mt = i / C::NTL, nt = i % C::NTL;
+      if constexpr (T::WIDE)
+        acc[mt][nt] = mfma_fp8_32x32x64(s0[C::NTL + mt], s1[C::NTL + mt], s0[nt], s1[nt], acc[mt][nt]);
+    };
+#pragma unroll
+    for (int q = 0; q < NOP; ++q) rdq(0, q, H0);
+#pragma unroll
+    for (int q = 0; q < NOP; ++q) rdq(1, q, H1);
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    const int wgrp = w >> 2;
+    if (wgrp == 1) lds_barrier();
+    const int nfull = Kb / BKB;
+    auto load_stage = [&](int p) {
+      if (p < nfull) {
+#pragma unroll
+        for (int j = 0; j < Q; ++j) issue1(j, p & 1, p * BKB);
+      } else if (p < nk) {
+#pragma unroll
+        for (int j = 0; j < Q; ++j) issue_half(j, p & 1, p * BKB);
+      }
+    };
+    auto step = [&](auto steady, auto odd, int h, u32x4 (&ha)[NOP], u32x4 (&hb)[NOP], u32x4 (&hc)[NOP], auto& hd) {
+      constexpr bool ST = decltype(steady)::value, ODD = decltype(odd)::value;
+      if (ODD) {
+        if (wgrp == 1) load_stage((h + 1) / 2 + 1);
+        else MK_WAIT_VMCNT(0);
+      } else if (wgrp == 0 && h > 0) {
+        load_stage(h / 2 + 1);
+      }
+      lds_barrier();
+      advance(ODD ? (((h + 1) >> 1) & 1 ? C::ST_BYTES : -C::ST_BYTES) : 0);   // to half-stage h + 1
+      const bool nxt = ST || h + 1 < nh;
+      __builtin_amdgcn_s_setprio(1);
+      if constexpr (T::WIDE) {
+        constexpr int NRD = 2 * NOP, RPM = (NRD + NMF - 1) / NMF;   // operand reads per MFMA
+#pragma unroll
+        for (int i = 0; i < NMF; ++i) {
+          mfqw(i, ha, hb);
+#pragma unroll
+          for (int q = i * RPM; q < (i + 1) * RPM && q < NRD; ++q)
+            if (nxt) rdq(q & 1, q >> 1, q & 1 ? hd : hc);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < NMF; ++i) {
+          mfq(i, ha);
+          if (i < NOP && nxt) rdq(0, i, hc);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int q = NMF; q < NOP; ++q)
+          if (nxt) rdq(0, q, hc);
+#pragma unroll
+        for (int i = 0; i < NMF; ++i) {
+          mfq(i, hb);
+          if (i < NOP && nxt) rdq(1, i, ha);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+#pragma unroll
+        for (int q = NMF; q < NOP; ++q)
+          if (nxt) rdq(1, q, ha);
+      }
+      __builtin_amdgcn_s_setprio(0);
+      __builtin_amdgcn_s_waitcnt(0xc07f);                 // half-stage h + 1 is in registers
+      if (!ODD && wgrp == 1) MK_WAIT_VMCNT(0);
+      lds_barrier();
+    };
+    using Yes = std::integral_constant<bool, true>;
+    using No = std::integral_constant<bool, false>;
+    int h = 0;
     if constexpr (T::WIDE) {
-      for (; it + 1 + D < nk; it += 2) {
-        step(Steady{}, it, H0, H1, H2, H3);
-        step(Steady{}, it + 1, H2, H3, H0, H1);
+      for (; h + 2 < nh; h += 2) {
+        step(Yes{}, No{}, h, H0, H1, H2, H3);
+        step(Yes{}, Yes{}, h + 1, H2, H3, H0, H1);
       }
-      for (; it < nk; it += 2) {
-        step(Tail{}, it, H0, H1, H2, H3);
-        if (it + 1 < nk) step(Tail{}, it + 1, H2, H3, H0, H1);
-      }
+      step(No{}, No{}, h, H0, H1, H2, H3);
+      if (h + 1 < nh) step(No{}, Yes{}, h + 1, H2, H3, H0, H1);
     } else {
-      for (; it + 2 + D < nk; it += 3) {
-        step(Steady{}, it, H0, H1, H2, H2);
-        step(Steady{}, it + 1, H2, H0, H1, H1);
-        step(Steady{}, it + 2, H1, H2, H0, H0);
+      for (; h + 6 < nh; h += 6) {
+        step(Yes{}, No{}, h, H0, H1, H2, H3);
+        step(Yes{}, Yes{}, h + 1, H2, H0, H1, H3);
+        step(Yes{}, No{}, h + 2, H1, H2, H0, H3);
+        step(Yes{}, Yes{}, h + 3, H0, H1, H2, H3);
+        step(Yes{}, No{}, h + 4, H2, H0, H1, H3);
+        step(Yes{}, Yes{}, h + 5, H1, H2, H0, H3);
       }
-      for (; it < nk; it += 3) {
-        step(Tail{}, it, H0, H1, H2, H2);
-        if (it + 1 < nk) step(Tail{}, it + 1, H2, H0, H1, H1);
-        if (it + 2 < nk) step(Tail{}, it + 2, H1, H2, H0, H0);
-      }
+      step(No{}, No{}, h, H0, H1, H2, H3);
+      if (h + 1 < nh) step(No{}, Yes{}, h + 1, H2, H0, H1, H3);
+      if (h + 2 < nh) step(No{}, No{}, h + 2, H1, H2, H0, H3);
+      if (h + 3 < nh) step(No{}, Yes{}, h + 3, H0, H1, H2, H3);
+      if (h + 4 < nh) step(No{}, No{}, h + 4, H2, H0, H1, H3);
+      if (h + 5 < nh) step(No{}, Yes{}, h + 5, H1, H2, H0, H3);
     }
     if (wgrp == 0) lds_barrier();
   } else if constexpr (C::LOOP == 2) {
@@ -1267,8 +1379,8 @@ int choose_cfg(const GemmArgs& g) {
     if (silu && fits(128, 128)) return 3;
   }
   struct Opt { int id, bm, bn; double eff; };
-  const Opt opts[6] = {{4, 256, 256, silu ? 1.05 : 1.25}, {2, 256, 128, 1.0}, {1, 256, 256, 0.9},
-                       {3, 128, 128, 0.85}, {5, 256, 192, 1.15}, {8, 256, 320, 1.14}};
+  const Opt opts[6] = {{4, 256, 256, silu ? 1.15 : 1.33}, {2, 256, 128, 1.0}, {1, 256, 256, 0.9},
+                       {3, 128, 128, 0.85}, {5, 256, 192, 1.25}, {8, 256, 320, 1.14}};
   int best = 2;
   double bt = 1e300;
   for (const Opt& o : opts) {

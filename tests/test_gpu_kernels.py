@@ -292,6 +292,30 @@ def test_gemm_short_problem_tiles(M, N, K):
     assert torch.equal(ops.gemm(ai, bi, "i32").double(), ai.double() @ bi.double().t())
 
 
+@pytest.mark.parametrize("N", [1536, 2048])
+@pytest.mark.parametrize("kb", [64, 128, 192, 384, 448, 1600, 4160])
+def test_gemm_ping_pong_stages(N, kb):
+    """256x192 and 256x256 ping-pong tiles (M = 8100, ragged): K of one half-stage up to 65, whole and half last
+    stages, over every remainder of the unrolled loop: int8 exact, bf16 within 64 eps sum|products| of
+    float64, fp8 within 1e-4 sum|products| (the fp8 unit's own precision)."""
+    from minicpm5_mk import ops
+
+    dev = _dev()
+    g = torch.Generator().manual_seed(N + kb)
+    M = 8100
+    print(f"[ping-pong] {M}x{N} K bytes {kb}", flush=True)
+    a = torch.randn(M, kb // 2, generator=g).to(BF16).to(dev)
+    b = torch.randn(N, kb // 2, generator=g).to(BF16).to(dev)
+    err = (ops.gemm(a, b, "f32").double() - a.double() @ b.double().t()).abs()
+    assert (err <= 64 * 2.0 ** -24 * (a.double().abs() @ b.double().abs().t())).all()
+    ai = torch.randint(-127, 128, (M, kb), generator=g, dtype=torch.int8).to(dev)
+    bi = torch.randint(-127, 128, (N, kb), generator=g, dtype=torch.int8).to(dev)
+    assert torch.equal(ops.gemm(ai, bi, "i32").double(), ai.double() @ bi.double().t())
+    af, bf = (t.to(dev) for t in _fp8_pair(M, N, kb, 5))
+    err = (ops.gemm(af, bf, "f32").double() - af.double() @ bf.double().t()).abs()
+    assert (err <= 1e-4 * (af.double().abs() @ bf.double().abs().t())).all()
+
+
 @pytest.mark.parametrize("epi", ["f32", "bf16", "res_f32add", "res_bf16add"])
 def test_gemm_wide_tile_rows_match(epi):
     """M = 8192, N = 2560 takes the 256x320 tile (one round of 256 CUs; 64x160 wave tiles, the epilogue

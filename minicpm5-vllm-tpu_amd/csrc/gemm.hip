@@ -100,7 +100,7 @@ using CfgX = GemmCfg<256, 256, 2, 4, 2, 1, 4>;
 using CfgN = GemmCfg<256, 192, 4, 2, 2, 1, 4>;
 // 256x320 block, 8 waves of 64x160: N = 2560 (the QKV projection at hd 128) in 8 column tiles, one round
 // of 256 CUs at M = 8192 where 256x192 tiles take 1.75 rounds; its epilogue stages 128 + 32 columns
-using CfgW = GemmCfg<256, 320, 4, 2, 4, 1, 1>;
+using CfgW = GemmCfg<256, 320, 4, 2, 2, 1, 4>;
 // Short problems (few tiles, each K loop latency-bound): 8-stage rings, seven stages of loads in flight.
 // 64x128 block, 32x64 per wave, one workgroup per CU (the 64x128 tile runs two stages per barrier: its waves
 // have few MFMAs per stage to cover a barrier)
@@ -526,6 +526,10 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
     // loads it in M(2p - 1) (4p - 1), group 0 in M(2p) (4p).  Its first reads are group 0's C(2p + 1), interval
     // 4p + 3: both groups wait for their loads at the end of 4p + 2 (group 0: M(2p + 1), group 1: C(2p)),
     // three to four intervals after issuing them.
+    // TWO: tiles whose accumulators leave no room for three operand sets keep two.  C(h) then reads its own
+    // second k-step and half-stage h + 1's first, so the last reads of stage p - 1 are in C(2p - 1) (4p - 1,
+    // 4p) and both groups load stage p + 1 in 4p + 1: group 0 in C(2p), group 1 in M(2p); waits as above.
+    constexpr bool TWO = !T::WIDE && 16 * C::MT * C::NTL + 12 * (C::MT + C::NTL) > 232;
     constexpr int NOP = C::MT + C::NTL;                   // operand registers per k-step: B then A
     u32x4 H0[NOP], H1[NOP], H2[NOP];
     u32x4 H3[T::WIDE ? NOP : 1];   // WIDE: half-stage h uses sets (H0, H1) or (H2, H3), all of it at once
@@ -556,7 +560,8 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
 #pragma unroll
     for (int q = 0; q < NOP; ++q) rdq(0, q, H0);
 #pragma unroll
-    for (int q = 0; q < NOP; ++q) rdq(1, q, H1);
+    for (int q = 0; q < NOP; ++q)
+      if (!TWO) rdq(1, q, H1);
     __builtin_amdgcn_s_waitcnt(0xc07f);
     const int wgrp = w >> 2;
     if (wgrp == 1) lds_barrier();
@@ -617,6 +622,36 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
       if (!ODD && wgrp == 1) MK_WAIT_VMCNT(0);
       lds_barrier();
     };
+    auto step2 = [&](auto steady, auto odd, int h) {
+      constexpr bool ST = decltype(steady)::value, ODD = decltype(odd)::value;
+      if (ODD) {
+        if (wgrp == 0) MK_WAIT_VMCNT(0);
+      } else if (wgrp == 1 && h > 0) {
+        load_stage(h / 2 + 1);
+      }
+      lds_barrier();
+      if (!ODD && wgrp == 0 && h > 0) load_stage(h / 2 + 1);
+      const bool nxt = ST || h + 1 < nh;
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int i = 0; i < NMF; ++i) {
+        mfq(i, H0);
+        if (i < NOP) rdq(1, i, H1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      static_assert(!TWO || NOP <= NMF, "operand reads under the MFMAs of one k-step");
+      advance(ODD ? (((h + 1) >> 1) & 1 ? C::ST_BYTES : -C::ST_BYTES) : 0);   // to half-stage h + 1
+#pragma unroll
+      for (int i = 0; i < NMF; ++i) {
+        mfq(i, H1);
+        if (i < NOP && nxt) rdq(0, i, H0);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      __builtin_amdgcn_s_setprio(0);
+      __builtin_amdgcn_s_waitcnt(0xc07f);
+      if (!ODD && wgrp == 1) MK_WAIT_VMCNT(0);
+      lds_barrier();
+    };
     using Yes = std::integral_constant<bool, true>;
     using No = std::integral_constant<bool, false>;
     int h = 0;
@@ -627,6 +662,13 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
       }
       step(No{}, No{}, h, H0, H1, H2, H3);
       if (h + 1 < nh) step(No{}, Yes{}, h + 1, H2, H3, H0, H1);
+    } else if constexpr (TWO) {
+      for (; h + 2 < nh; h += 2) {
+        step2(Yes{}, No{}, h);
+        step2(Yes{}, Yes{}, h + 1);
+      }
+      step2(No{}, No{}, h);
+      if (h + 1 < nh) step2(No{}, Yes{}, h + 1);
     } else {
       for (; h + 6 < nh; h += 6) {
         step(Yes{}, No{}, h, H0, H1, H2, H3);

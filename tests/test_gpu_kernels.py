@@ -292,10 +292,10 @@ def test_gemm_short_problem_tiles(M, N, K):
     assert torch.equal(ops.gemm(ai, bi, "i32").double(), ai.double() @ bi.double().t())
 
 
-@pytest.mark.parametrize("N", [1536, 2048])
+@pytest.mark.parametrize("N", [1536, 2048, 2560])
 @pytest.mark.parametrize("kb", [64, 128, 192, 384, 448, 1600, 4160])
 def test_gemm_ping_pong_stages(N, kb):
-    """256x192 and 256x256 ping-pong tiles (M = 8100, ragged): K of one half-stage up to 65, whole and half last
+    """256x192, 256x256 and 256x320 (bf16, int8) ping-pong tiles (M = 8100, ragged): K of one half-stage up to 65, whole and half last
     stages, over every remainder of the unrolled loop: int8 exact, bf16 within 64 eps sum|products| of
     float64, fp8 within 1e-4 sum|products| (the fp8 unit's own precision)."""
     from minicpm5_mk import ops

@@ -51,7 +51,8 @@ struct GemmCfg {
   static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, NST = NST_, OCC = OCC_;
   // main loop: 0 split k-step pipeline, 1 ping-pong (two wave groups, operand prefetch), 2 two stages
   // per barrier with the operands read half a stage ahead, 3 128-byte stages with the operands read a whole
-  // stage ahead and loader waves, 4 ping-pong over 128-byte stages in two slots
+  // stage ahead and loader waves, 4 ping-pong over 128-byte stages in two slots, 5 whole-stage operand sets
+  // on 128-byte stages in two slots
   static constexpr int LOOP = LOOP_;
   static constexpr int NW = WGM * WGN;                    // compute waves
   static constexpr int LW = LOOP == 3 ? NW : 0;           // loader waves
@@ -112,6 +113,10 @@ using CfgE = GemmCfg<64, 128, 2, 2, 8, 1, 2>;
 // twice the bytes are in flight when the weights are cold (1B down at M = 256, us warm / cold: 64x128 with
 // 64-byte stages 29.1 / 45.6, this 64x128 24.4 / 33.6, 64x64 17.8 / 23.2, 32x64 17.8 / 19.3).
 using CfgD = GemmCfg<128, 128, 2, 2, 5, 1, 3>;
+// Mid-size problems on whole cache lines, two workgroups per CU: 192x128 block, 96x64 per wave, and 128x128,
+// 64x64 per wave
+using CfgP = GemmCfg<192, 128, 2, 2, 2, 2, 5>;
+using CfgQ = GemmCfg<128, 128, 2, 2, 2, 2, 5>;
 using CfgF = GemmCfg<64, 64, 2, 2, 5, 2, 3>;
 using CfgG = GemmCfg<32, 64, 1, 2, 10, 1, 3>;
 using CfgH = GemmCfg<64, 128, 2, 2, 6, 1, 3>;
@@ -686,6 +691,54 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
       if (h + 5 < nh) step(No{}, Yes{}, h + 5, H1, H2, H0, H3);
     }
     if (wgrp == 0) lds_barrier();
+  } else if constexpr (C::LOOP == 5) {
+    // Pairs of workgroups per CU on whole-line stages, two slots each.  A stage's operands (four k-steps) are
+    // all read into registers, the MFMAs starting with the first; when every wave has them (first barrier) the
+    // slot takes the stage after next, under the rest of the MFMAs; the second barrier makes the next stage
+    // visible.  The other workgroup of the CU issues while this one waits.
+    u32x4 za[4][C::MT], zb[4][C::NTL];
+    constexpr int HEAD = 3 * NMF;   // MFMAs before the first barrier: the last k-step's reads land under them
+    for (int it = 0; it < nk; ++it) {
+      const char* S = smem + (it & 1) * C::ST_BYTES;
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        const int x = 16 * ((2 * ks + half) ^ sw);
+#pragma unroll
+        for (int nt = 0; nt < C::NTL; ++nt) zb[ks][nt] = *reinterpret_cast<const u32x4*>(S + bro + x + nt * 32 * BKB);
+#pragma unroll
+        for (int mt = 0; mt < C::MT; ++mt) za[ks][mt] = *reinterpret_cast<const u32x4*>(S + aro + x + mt * 32 * BKB);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+      auto mfmas = [&](int i0, int i1) {
+#pragma unroll
+        for (int i = 0; i < 4 * NMF; ++i) {
+          if (i < i0 || i >= i1) continue;
+          const int ks = i / NMF;
+          if constexpr (T::WIDE) {
+            // k-steps 0 and 1 first, 2 and 3 after the barrier
+            if (ks == 0 || ks == 3) mfw(i % NMF, za[ks & 2], zb[ks & 2], za[(ks & 2) + 1], zb[(ks & 2) + 1]);
+          } else {
+            mf(i % NMF, za[ks], zb[ks]);
+          }
+        }
+      };
+      mfmas(0, HEAD);
+      __builtin_amdgcn_sched_barrier(0);
+      if (it + 2 < nk) {
+        __builtin_amdgcn_s_waitcnt(0xc07f);
+        lds_barrier();
+#pragma unroll
+        for (int j = 0; j < Q; ++j) issue1(j, it & 1, (it + 2) * BKB);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+      mfmas(HEAD, 4 * NMF);
+      __builtin_amdgcn_sched_barrier(0);
+      if (it + 1 < nk) {
+        if (it + 2 < nk) wait_stages(std::integral_constant<int, 1>{});
+        else wait_stages(W0{});
+        lds_barrier();
+      }
+    }
   } else if constexpr (C::LOOP == 2) {
     // Two stages per iteration and one barrier.  Operand sets X0 .. X3 hold (stage it, k-step 0),
     // (it, 1), (it + 1, 0), (it + 1, 1).  X2 and X3 are read at the top of the iteration, under the
@@ -1376,7 +1429,9 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(GemmArgs g, int spli
 // per tile, except for the SiLU epilogue, whose VALU work is hidden better by two co-resident
 // 256x128 workgroups.  The 256x320 tile's 1.14: the QKV shape M = 8192, N = 2560, K = 1536 (dequantising
 // epilogue, no routing) takes 40.9 us on it, 48.6 us on 256x192 tiles (1.75 rounds) and 52.3 us on
-// 256x256 ones (1.25 rounds).
+// 256x256 ones (1.25 rounds); with 128-byte stages 37.5 against 39.5 us, and 41.9 on 256x192.  The SiLU 256x256
+// tile's 1.10 (1.15 fits its own times, 125 us for the 1B gate/up at M = 8192 against 130 on 256x128 pairs):
+// inside the model the pairs take 127 us there against 130, and the attention next to them 231 against 240.
 int choose_cfg(const GemmArgs& g) {
   const bool silu = g.epi == Epi::DQ_SILU || g.epi == Epi::DQ_SILU_F32A || g.epi == Epi::SILU_BF16;
   // 5 and 8 (96- and 160-column waves) cannot hold whole [gate | up] blocks
@@ -1385,15 +1440,15 @@ int choose_cfg(const GemmArgs& g) {
   const bool wide320 = !silu && g.in != GemmIn::F8;
   const int kb = g.K * (g.in == GemmIn::BF16 ? 2 : 1);   // bytes
   const bool line = kb % 128 == 0;                        // whole 128-byte stages
-  // 5, 8, 9, 10: waves without whole [gate | up] blocks; 6, 9 - 12: 128-byte stages
+  // 5, 8, 9, 10: waves without whole [gate | up] blocks; 12: built for SiLU alone; 6, 9 - 13: whole lines
   auto ok = [&](int id) {
     if (id == 8) return wide320;
-    if (silu) return id >= 1 && id <= 7 && id != 5 && id != 6;
-    return id >= 1 && id <= 11 && (line || !(id == 6 || id >= 9));
+    if (silu) return (id >= 1 && id <= 7 && id != 5 && id != 6) || (line && id == 12);
+    return id >= 1 && id <= 13 && id != 12 && (line || !(id == 6 || id >= 9));
   };
   if (ok(g.cfg)) return g.cfg;
   static const int forced = [] {
-    const char* e = std::getenv("MK_GEMM_CFG");   // tuning override: 1 .. 8
+    const char* e = std::getenv("MK_GEMM_CFG");   // tuning override: 1 .. 13
     return e ? std::atoi(e) : 0;
   }();
   if (ok(forced)) return forced;
@@ -1418,15 +1473,21 @@ int choose_cfg(const GemmArgs& g) {
     }
     if (kb >= 1024 && fits(64, 128)) return 7;
     if (!silu && line && lines >= 32 && fits(128, 128)) return 6;
+    // up to two 128x128 workgroups per CU: 1B down at M = 4096 72.3 -> 60.4 us (before: one 256x128 tile per CU),
+    // O at M = 3072 34.5 -> 29.5, QKV at M = 2500 19.4 -> 18.0, 2B down at M = 4096 103 -> 96.9 (256x256 109)
+    if (!silu && line && !fits(128, 128) && (long)((g.M + 127) / 128) * ((g.N + 127) / 128) <= 512) return 13;
     if (silu && fits(128, 128)) return 3;
   }
   struct Opt { int id, bm, bn; double eff; };
-  const Opt opts[6] = {{4, 256, 256, silu ? 1.15 : 1.33}, {2, 256, 128, 1.0}, {1, 256, 256, 0.9},
-                       {3, 128, 128, 0.85}, {5, 256, 192, 1.25}, {8, 256, 320, 1.14}};
+  const Opt opts[7] = {{4, 256, 256, silu ? 1.10 : 1.33}, {2, 256, 128, 1.0}, {1, 256, 256, 0.9},
+                       {3, 128, 128, 0.85}, {5, 256, 192, 1.25}, {8, 256, 320, 1.14}, {12, 192, 128, 1.0}};
   int best = 2;
   double bt = 1e300;
   for (const Opt& o : opts) {
     if ((silu && (o.id == 3 || o.id == 5)) || (!wide320 && o.id == 8)) continue;   // 3: never faster; 5, 8: no SiLU
+    // 192x128 pairs fill rounds the larger tiles leave half empty: 2B gate/up at M = 1536 52.0 -> 43.9 us, at
+    // M = 3072 88.4 -> 82.6, 1B gate/up at M = 6000 103 -> 96.7
+    if (o.id == 12 && !(silu && line)) continue;
     const double tiles = (double)((g.M + o.bm - 1) / o.bm) * ((g.N + o.bn - 1) / o.bn);
     const double t = std::ceil(tiles / 256.0) * o.bm * o.bn / o.eff;
     if (t < bt * 0.999) {
@@ -1503,6 +1564,12 @@ void launch_t(const GemmArgs& g, hipStream_t st) {
       break;
     case 11:
       if constexpr (!silu) launch_c<CfgH, IN, EPI>(g, st);
+      break;
+    case 12:
+      if constexpr (silu) launch_c<CfgP, IN, EPI>(g, st);
+      break;
+    case 13:
+      if constexpr (!silu) launch_c<CfgQ, IN, EPI>(g, st);
       break;
     default: launch_c<CfgM, IN, EPI>(g, st); break;
   }

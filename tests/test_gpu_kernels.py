@@ -13,7 +13,7 @@
   * activation quantisation in the fp8d / int8 / fp8 modes: bit-exact codes (the static modes with
     RMSNorm round x * rstd to bf16, so an rstd one f32 ulp off may move a code by one step: at most
     0.1% of codes, each by one step); f32 -> e4m3 conversion bit-exact over every finite bf16 value.
-  * fp8 GEMM: v_mfma_f32_32x32x16_fp8_fp8 sums its 16 products at reduced internal precision (measured
+  * fp8 GEMM: the fp8 MFMAs (v_mfma_f32_32x32x64_f8f6f4) sum their products at reduced internal precision (measured
     on MI355X: max error 2.4e-5 of sum|products| at K = 64, 1.5e-6 at K = 4608, zero when the products
     span few binades), so the bound is 1e-4 * sum|products| of the exact (float64) result; dequant
     epilogues within 1 bf16 ulp + that bound.
@@ -101,13 +101,14 @@ def test_attention_deterministic():
     assert torch.equal(a, b)
 
 
-@pytest.mark.parametrize("B,S,hd", [(2, 4096, 128), (4, 2048, 96), (3, 2048, 128)])
+@pytest.mark.parametrize("B,S,hd", [(2, 4096, 128), (4, 2048, 96), (3, 2048, 128), (4, 768, 96), (4, 768, 64)])
 def test_attention_batch_invariant(B, S, hd):
     """Each sequence of a batch equals the same sequence run alone, bit for bit.  (2, 4096) and
     (4, 2048) launch 256 tile pairs (B * 2 kv heads * S / 64) and take the static pair mapping;
     (3, 2048) launches 384 items on 256 persistent workgroups, so workgroups take several items and
     drain the other kv head's queue; the single-sequence runs have no more items than CUs and take the
-    direct mapping (workgroup i computes item i, no queue)."""
+    direct mapping (workgroup i computes item i, no queue).  (4, 768) launches 192 items of 8 waves, its
+    single sequences items of 4 waves."""
     from minicpm5_mk import ops
     from minicpm5_mk.mk_weights import rope_tables
 
@@ -290,6 +291,47 @@ def test_gemm_short_problem_tiles(M, N, K):
     ai = torch.randint(-127, 128, (M, 2 * K), generator=g, dtype=torch.int8).to(dev)
     bi = torch.randint(-127, 128, (N, 2 * K), generator=g, dtype=torch.int8).to(dev)
     assert torch.equal(ops.gemm(ai, bi, "i32").double(), ai.double() @ bi.double().t())
+
+
+@pytest.mark.parametrize("M,N,K", [(2900, 1528, 64), (4000, 1536, 128), (2300, 2008, 1536), (2300, 2008, 192)])
+def test_gemm_mid_size_tiles(M, N, K):
+    """128x128 workgroup pairs (257 .. 512 tiles; K loops of one, two, three and many stages, ragged rows and
+    columns): bf16 rows bitwise equal to those of a product of 9000 rows and within 64 eps sum|products| of
+    float64, int8 exact, fp8 within 1e-4 sum|products|."""
+    from minicpm5_mk import ops
+
+    dev = _dev()
+    g = torch.Generator().manual_seed(M + K)
+    print(f"[mid tiles] {M}x{N}x{K}", flush=True)
+    a = torch.randn(9000, K, generator=g).to(BF16).to(dev)
+    b = (torch.randn(N, K, generator=g) * 0.02).to(BF16).to(dev)
+    out = ops.gemm(a[:M].contiguous(), b, "f32")
+    assert torch.equal(out.view(torch.int32), ops.gemm(a, b, "f32")[:M].view(torch.int32))
+    ref = a[:M].double() @ b.double().t()
+    assert ((out.double() - ref).abs() <= 64 * 2.0 ** -24 * (a[:M].double().abs() @ b.double().abs().t())).all()
+    ai = torch.randint(-127, 128, (M, 2 * K), generator=g, dtype=torch.int8).to(dev)
+    bi = torch.randint(-127, 128, (N, 2 * K), generator=g, dtype=torch.int8).to(dev)
+    assert torch.equal(ops.gemm(ai, bi, "i32").double(), ai.double() @ bi.double().t())
+    af, bf = (t.to(dev) for t in _fp8_pair(M, N, 2 * K, 6))
+    err = (ops.gemm(af, bf, "f32").double() - af.double() @ bf.double().t()).abs()
+    assert (err <= 1e-4 * (af.double().abs() @ bf.double().abs().t())).all()
+
+
+@pytest.mark.parametrize("M,N,K", [(200, 9216, 1536), (1500, 12288, 256), (1400, 12288, 128), (5990, 9216, 384)])
+def test_gate_up_tiles_match(M, N, K):
+    """SiLU epilogue on the tiles chosen for short and mid-size gate/up problems (128x128, 192x128 pairs with an
+    even, a single and an odd number of stages): rows bitwise equal to the same rows of a product of 8192."""
+    from minicpm5_mk import ops
+
+    dev = _dev()
+    g = torch.Generator().manual_seed(M + N)
+    print(f"[gate/up tiles] {M}x{N}x{K}", flush=True)
+    a = torch.randint(-127, 128, (8192, K), generator=g, dtype=torch.int8).to(dev)
+    b = torch.randint(-127, 128, (N, K), generator=g, dtype=torch.int8).to(dev)
+    rs, cs = (torch.rand(8192, generator=g) * 1e-2).to(dev), (torch.rand(N, generator=g) * 1e-2).to(dev)
+    big = ops.gemm(a, b, "dq_silu", rs=rs, cs=cs)
+    out = ops.gemm(a[:M].contiguous(), b, "dq_silu", rs=rs[:M].contiguous(), cs=cs)
+    assert torch.equal(out.view(torch.int16), big[:M].view(torch.int16))
 
 
 @pytest.mark.parametrize("N", [1536, 2048, 2560])

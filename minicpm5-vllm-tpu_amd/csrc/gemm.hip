@@ -214,7 +214,8 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
   using T = Mma<IN>;
   using Acc = typename T::Acc;
   constexpr int BKB = C::BKB;
-  __shared__ __attribute__((aligned(1024))) char smem[C::NST * C::ST_BYTES];
+  constexpr int PF_BYTES = C::LOOP == 4 ? 512 : 0;        // landing area of the L2 prefetches
+  __shared__ __attribute__((aligned(1024))) char smem[C::NST * C::ST_BYTES + PF_BYTES];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int w = __builtin_amdgcn_readfirstlane(tid >> 6);   // wave index, kept in an SGPR
@@ -571,6 +572,27 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
     const int wgrp = w >> 2;
     if (wgrp == 1) lds_barrier();
     const int nfull = Kb / BKB;
+    // Prefetch into L2, two stages ahead of the loads.  The workgroups of an XCD walk K together, so every
+    // stage is a first touch for all of them, and with weights cold in HBM it takes longer to come than the
+    // loads have.  Waves 0 and 1 touch 64 lines each, one dword of a line, dropped into a scratch area: a
+    // quarter of the A rows (by column tile) and one of the BN / 64 parts of the B rows (by row tile), the
+    // neighbours the rest.
+    const bool pfw = w < 2;
+    uint32_t pfo;
+    {
+      const int tm = m0 / BM, tn = n0 / BN;
+      const uint32_t ra = (uint32_t)min(m0 + 64 * (tn % (BM / 64)) + lane, g.M - 1) * (uint32_t)lda;
+      const uint32_t rb = (uint32_t)min(n0 + 64 * (tm % (BN / 64)) + lane, g.N - 1) * (uint32_t)ldb;
+      pfo = w == 0 ? ra : rb;
+    }
+    auto prefetch = [&](int p) {
+      if (pfw && p < nk) copy4_to_lds(w == 0 ? rA : rB, pfo, (uint32_t)(p * BKB), smem + C::NST * C::ST_BYTES + w * 256);
+    };
+    // group 0's wait for its loads: the prefetch issued after them may be outstanding
+    auto wait_loads = [&](int p) {
+      if (pfw && p + 3 < nk) MK_WAIT_VMCNT(1);
+      else MK_WAIT_VMCNT(0);
+    };
     auto load_stage = [&](int p) {
       if (p < nfull) {
 #pragma unroll
@@ -584,9 +606,10 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
       constexpr bool ST = decltype(steady)::value, ODD = decltype(odd)::value;
       if (ODD) {
         if (wgrp == 1) load_stage((h + 1) / 2 + 1);
-        else MK_WAIT_VMCNT(0);
-      } else if (wgrp == 0 && h > 0) {
-        load_stage(h / 2 + 1);
+        else wait_loads(h / 2);
+      } else if (wgrp == 0) {
+        if (h > 0) load_stage(h / 2 + 1);
+        prefetch(h / 2 + 3);
       }
       lds_barrier();
       advance(ODD ? (((h + 1) >> 1) & 1 ? C::ST_BYTES : -C::ST_BYTES) : 0);   // to half-stage h + 1
@@ -630,12 +653,15 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
     auto step2 = [&](auto steady, auto odd, int h) {
       constexpr bool ST = decltype(steady)::value, ODD = decltype(odd)::value;
       if (ODD) {
-        if (wgrp == 0) MK_WAIT_VMCNT(0);
+        if (wgrp == 0) wait_loads(h / 2);
       } else if (wgrp == 1 && h > 0) {
         load_stage(h / 2 + 1);
       }
       lds_barrier();
-      if (!ODD && wgrp == 0 && h > 0) load_stage(h / 2 + 1);
+      if (!ODD && wgrp == 0) {
+        if (h > 0) load_stage(h / 2 + 1);
+        prefetch(h / 2 + 3);
+      }
       const bool nxt = ST || h + 1 < nh;
       __builtin_amdgcn_s_setprio(1);
 #pragma unroll

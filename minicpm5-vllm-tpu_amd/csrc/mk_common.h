@@ -147,6 +147,11 @@ __device__ inline void copy16_to_lds(__amdgpu_buffer_rsrc_t r, uint32_t voff, ui
   __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr)dst, 16, voff, soff, 0, 0);
 }
 
+// 4 bytes per lane (dst + 4 l), the offset split the same way.
+__device__ inline void copy4_to_lds(__amdgpu_buffer_rsrc_t r, uint32_t voff, uint32_t soff, char* dst) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_ptr)dst, 4, voff, soff, 0, 0);
+}
+
 // acc + lo(w) + hi(w) for a packed bf16 pair (v_dot2_f32_bf16 with (1, 1))
 __device__ inline float dot2_bf16_sum(uint32_t w, float acc) {
   return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(bf16x2, w), __builtin_bit_cast(bf16x2, 0x3f803f80u),

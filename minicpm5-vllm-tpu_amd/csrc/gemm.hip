@@ -49,10 +49,9 @@ constexpr int epi_chunk(int ntl, int ew, int nw, int ring_bytes) {
 template <int BM_, int BN_, int WGM_, int WGN_, int NST_, int OCC_, int LOOP_ = 0>
 struct GemmCfg {
   static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, NST = NST_, OCC = OCC_;
-  // main loop: 0 split k-step pipeline, 1 ping-pong (two wave groups, operand prefetch), 2 two stages
-  // per barrier with the operands read half a stage ahead, 3 128-byte stages with the operands read a whole
-  // stage ahead and loader waves, 4 ping-pong over 128-byte stages in two slots, 5 whole-stage operand sets
-  // on 128-byte stages in two slots
+  // main loop: 0 split k-step pipeline; 2 two stages per barrier, the operands read half a stage ahead;
+  // 3 128-byte stages, loader waves, the operands read a whole stage ahead; 4 ping-pong (two wave groups) over
+  // 128-byte stages in two slots; 5 whole-stage operand sets, 128-byte stages in two slots
   static constexpr int LOOP = LOOP_;
   static constexpr int NW = WGM * WGN;                    // compute waves
   static constexpr int LW = LOOP == 3 ? NW : 0;           // loader waves
@@ -62,29 +61,27 @@ struct GemmCfg {
   static constexpr int BKB = stage_kb(LOOP);
   static constexpr int A_BYTES = BM * BKB, ST_BYTES = (BM + BN) * BKB;
   // a stage is NL blocks of RPB rows x BKB bytes (1 KB, one async-load instruction): A blocks 0 .. NA-1,
-  // then B blocks; block b is loaded by wave b % NW.  Waves w < NL % NW load QH blocks, the rest QL.
+  // then B blocks; block b is loaded by wave b % NW, Q blocks per wave.
   static constexpr int RPB = 1024 / BKB, CPR = BKB / 16;   // rows per block, 16-byte chunks per row
   static constexpr int NA = BM / RPB, NL = (BM + BN) / RPB;
-  static constexpr int QL = NL / NW, QH = (NL + NW - 1) / NW, NQH = NL % NW == 0 ? NW : NL % NW;
+  static constexpr int Q = NL / NW;
   static constexpr int EW = WN % 64 == 0 ? 64 : 32;       // epilogue pass width (columns)
   static constexpr int ECH = epi_chunk(NTL, EW, NW, NST * ST_BYTES);   // 32-column tiles per staging chunk
   static constexpr int NECH = (NTL + ECH - 1) / ECH;
   static constexpr int EROW = ECH * 32 * 4 + 16;          // epilogue LDS row (f32 + pad)
   static_assert(BM % RPB == 0 && BN % RPB == 0 && NA % NW == 0, "load split: A blocks evenly over the waves");
-  static_assert(LOOP != 4 || (NW == 8 && NST == 2 && NL % NW == 0), "two-slot ping-pong: two groups of four waves");
-  static_assert(LOOP == 1 || NL % NW == 0, "split k-step loop: the same load count on every wave");
+  static_assert(LOOP != 4 || (NW == 8 && NST == 2), "two-slot ping-pong: two groups of four waves");
+  static_assert(NL % NW == 0, "the same load count on every wave");
   static_assert(NW * 32 * EROW <= NST * ST_BYTES, "epilogue staging fits in the ring");
   static_assert(WN % 32 == 0, "wave tile width");
   // ping-pong: waves w and w + 4 share a SIMD and belong to groups 0 and 1; each group loads a uniform
   // number of blocks per stage
   static_assert(LOOP != 2 || NST >= 5, "two-stage loop: stages it + 2, it + 3 land while it + 4 .. are in flight");
-  static_assert(LOOP != 3 || (NL % NW == 0 && NST >= 3), "whole-stage loop: uniform loads, two stages in flight");
-  static_assert(LOOP != 1 || (NW == 8 && NST >= 3 && NQH % 4 == 0),
-                "ping-pong needs two groups of four waves with uniform loads and two stages in flight");
+  static_assert(LOOP != 3 || NST >= 3, "whole-stage loop: two stages in flight");
   // Lean addressing for ping-pong tiles whose accumulators and three operand sets nearly fill the 256
   // registers of a wave: the async-load lane offsets that follow from others are recomputed where
   // they are used instead of being held through the main loop (held, they spilled into the loop).
-  static constexpr bool LEAN = (LOOP == 1 || LOOP == 4) && 16 * MT * NTL + 12 * (MT + NTL) > (LOOP == 4 ? 190 : 232);
+  static constexpr bool LEAN = LOOP == 4 && 16 * MT * NTL + 12 * (MT + NTL) > 190;
 };
 // 256x256 block, 128x128 per wave (accumulators in AGPRs), one workgroup per CU
 using CfgL = GemmCfg<256, 256, 2, 2, 3, 1, 0>;
@@ -239,9 +236,8 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
   const int m0 = (first_m + wig % gsz) * C::BM, n0 = (wig / gsz) * C::BN;
   const int lda = g.lda * T::ESZ, ldb = g.ldb * T::ESZ;   // bytes
   const int Kb = g.K * T::ESZ;
-  // async-load instructions per wave per stage: QH on waves w < NQH (ping-pong group 0 when uneven)
-  constexpr int Q = C::QH;
-  const bool qfull = C::QH == C::QL || w < C::NQH;
+  constexpr int Q = C::Q;   // async-load instructions per wave per stage
+
 
   // this lane's async-load sources: block b = w + NW j, rows RPB (b or b - NA) + lane / CPR of A or B, as
   // 32-bit byte offsets from the operand base (the base and the K offset stay scalar); rows past M / N
@@ -290,7 +286,7 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
   auto issue1 = [&](int j, int st, int kb) {
     char* dst = smem + st * C::ST_BYTES + (lw + C::NW * j) * 1024;
     if (j < JA) copy16_to_lds(rA, voff(j), (uint32_t)kb, dst);
-    else if (j < C::QL || qfull) copy16_to_lds(rB, voff(j), (uint32_t)kb, dst);
+    else copy16_to_lds(rB, voff(j), (uint32_t)kb, dst);
   };
   // A last stage of half the K bytes (LOOP 4): its other half would read past the row (unused), and past the
   // last row out of the buffer, so the K offset goes where the range check sees it (out of range: zeros).
@@ -300,9 +296,8 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
   // wait until at most `n` stages of this wave's async loads are outstanding
   auto wait_stages = [&](auto nc) {
     constexpr int n = decltype(nc)::value;
-    static_assert(n * C::QH <= 63, "vmcnt counts at most 63 loads");
-    if (C::QH == C::QL || qfull) MK_WAIT_VMCNT(n * C::QH);
-    else MK_WAIT_VMCNT(n * C::QL);
+    static_assert(n * Q <= 63, "vmcnt counts at most 63 loads");
+    MK_WAIT_VMCNT(n * Q);
   };
   using W0 = std::integral_constant<int, 0>;
   // wait until at most min(n, left) stages are outstanding (left: stages there are beyond the one waited for)
@@ -422,111 +417,17 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
   // Materialize the epilogue's kernel arguments now: a scalar load still pending inside the loop would
   // turn every LDS wait there into lgkmcnt(0) (scalar loads return out of order).
   asm volatile("" ::"s"(g.out), "s"(g.res), "s"(g.rs), "s"(g.cs), "s"(g.aux), "s"(g.ldo), "s"(g.ldr));
-  if constexpr (C::LOOP == 1) {
-    // Ping-pong.  The waves form two groups (wm = 0, 1) with one wave of each on every SIMD, and each
-    // iteration is a memory phase M (async loads of the stage NST - 1 ahead) and a compute phase C
-    // (the stage's MFMAs, with the next stage's operands read from LDS into registers alongside), each
-    // closed by a barrier.  Group 1 starts one barrier late, so on every SIMD one wave issues MFMAs
-    // while the other is in its memory phase or waiting at the barrier.
-    // Operands live in a ring of three k-step register sets: stage s uses (2s, 2s + 1) mod 3, and
-    // stage s + 1's k-step 0 goes to the free set, its k-step 1 to the set stage s's k-step 0 used.
-    // Stage s + 1 must be visible when group 0 starts C(s): group 0 waits for its loads of stage s + 1
-    // at the end of M(s), group 1 at the end of C(s - 1).  A stage's slot is refilled in M(s + 1) of
-    // the stage NST ahead, after both groups finished reading it in their C(s - 1).
-    constexpr int D = C::NST - 1;
-    constexpr int NOP = C::MT + C::NTL;                   // operand registers per k-step: B then A
-    u32x4 H0[NOP], H1[NOP], H2[NOP];
-    static_assert(!T::WIDE, "one k-step per operand set");
-    auto rdq = [&](const char* Sb, int ks, int q, u32x4 (&dst)[NOP]) {
-      if (q < C::NTL) dst[q] = *reinterpret_cast<const u32x4*>(Sb + (ks ? bo1 : bo0) + q * 32 * BKB);
-      else dst[q] = *reinterpret_cast<const u32x4*>(Sb + (ks ? ao1 : ao0) + (q - C::NTL) * 32 * BKB);
-    };
-    auto mfq = [&](int i, const u32x4 (&src)[NOP]) {
-      const int mt = i / C::NTL, nt = i % C::NTL;
-      acc[mt][nt] = T::run(src[C::NTL + mt], src[nt], acc[mt][nt]);
-    };
-    // stages 0 and 1 visible; stage 0 in H0 / H1
-    if (nk >= D) wait_stages(std::integral_constant<int, D - 2>{});
-    else wait_stages(W0{});
-    lds_barrier();
-#pragma unroll
-    for (int q = 0; q < NOP; ++q) rdq(smem, 0, q, H0);
-#pragma unroll
-    for (int q = 0; q < NOP; ++q) rdq(smem, 1, q, H1);
-    __builtin_amdgcn_s_waitcnt(0xc07f);
-    // ping-pong group of this wave: waves w and w + 4 share a SIMD; group 0 loads QH blocks per stage,
-    // group 1 QL
-    const int wgrp = w >> 2;
-    if (wgrp == 1) lds_barrier();
-    int cur = 0;
-    // `steady` instances (stage it + D exists) have no runtime conditions, so the compute phase stays one
-    // basic block instead of a branch around every operand read
-    auto step = [&](auto steady, int it, u32x4 (&ha)[NOP], u32x4 (&hb)[NOP], u32x4 (&hc)[NOP]) {
-      constexpr bool ST = decltype(steady)::value;
-      // M(it): async loads of stage it + D into the slot of stage it - 1
-      const bool pre = ST || it + D < nk;
-      if (pre) {
-        const int nslot = cur == 0 ? C::NST - 1 : cur - 1;
-#pragma unroll
-        for (int j = 0; j < Q; ++j) issue1(j, nslot, (it + D) * BKB);
-      }
-      if (wgrp == 0 && (ST || it + 1 < nk)) {
-        if (pre) MK_WAIT_VMCNT((D - 1) * C::QH);
-        else MK_WAIT_VMCNT(0);
-      }
-      lds_barrier();
-      // C(it): MFMAs of stage it, reads of stage it + 1
-      const int s1 = cur == C::NST - 1 ? 0 : cur + 1;
-      const char* S1 = smem + s1 * C::ST_BYTES;
-      const bool nxt = ST || it + 1 < nk;
-      __builtin_amdgcn_s_setprio(1);
-#pragma unroll
-      for (int i = 0; i < NMF; ++i) {
-        mfq(i, ha);
-        if (i < NOP && nxt) rdq(S1, 0, i, hc);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-#pragma unroll
-      for (int q = NMF; q < NOP; ++q)
-        if (nxt) rdq(S1, 0, q, hc);
-#pragma unroll
-      for (int i = 0; i < NMF; ++i) {
-        mfq(i, hb);
-        if (i < NOP && nxt) rdq(S1, 1, i, ha);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-#pragma unroll
-      for (int q = NMF; q < NOP; ++q)
-        if (nxt) rdq(S1, 1, q, ha);
-      __builtin_amdgcn_s_setprio(0);
-      __builtin_amdgcn_s_waitcnt(0xc07f);                 // lgkmcnt(0): stage it + 1 is in registers
-      if (wgrp == 1 && (ST || it + 2 < nk)) {
-        if (pre) MK_WAIT_VMCNT((D - 2) * C::QL);
-        else MK_WAIT_VMCNT(0);
-      }
-      lds_barrier();
-      cur = s1;
-    };
-    using Steady = std::integral_constant<bool, true>;
-    using Tail = std::integral_constant<bool, false>;
-    int it = 0;
-    for (; it + 2 + D < nk; it += 3) {
-      step(Steady{}, it, H0, H1, H2);
-      step(Steady{}, it + 1, H2, H0, H1);
-      step(Steady{}, it + 2, H1, H2, H0);
-    }
-    for (; it < nk; it += 3) {
-      step(Tail{}, it, H0, H1, H2);
-      if (it + 1 < nk) step(Tail{}, it + 1, H2, H0, H1);
-      if (it + 2 < nk) step(Tail{}, it + 2, H1, H2, H0);
-    }
-    if (wgrp == 0) lds_barrier();
-  } else if constexpr (C::LOOP == 4) {
+  if constexpr (C::LOOP == 4) {
     // Ping-pong over 128-byte stages in two LDS slots: whole cache lines per row, two half-stages (64 bytes of
     // K) of MFMAs per stage.  With 64-byte slices every load of a line's other half, a stage later, misses
     // the 32 KB L1 again and L2 delivers each line twice.
-    // Half-stage h = 2 p + (0 or 1) of stage p; phases M(h), C(h) per half-stage as in the loop above, C(h)
-    // reading half-stage h + 1.  Number the barrier intervals so that group 0 runs M(h) in 2h and C(h) in
+    // The waves form two groups with one wave of each on every SIMD (waves w and w + 4).  Half-stage
+    // h = 2 p + (0 or 1) of stage p has a memory phase M(h) (async loads) and a compute phase C(h) (its MFMAs,
+    // half-stage h + 1 read from LDS into registers alongside), each closed by a barrier.  Group 1 starts one
+    // barrier late, so on every SIMD one wave issues MFMAs while the other is in its memory phase or waiting.
+    // Operands live in a ring of three k-step register sets: C(h) reads half-stage h + 1's k-step 0 into the
+    // free set and its k-step 1 into the set h's k-step 0 used.
+    //  Number the barrier intervals so that group 0 runs M(h) in 2h and C(h) in
     // 2h + 1, group 1 M(h) in 2h + 1 and C(h) in 2h + 2.  Stage p - 1's last reads (half 2p - 1) are in
     // C(2p - 2): intervals 4p - 3 and 4p - 2, so its slot takes stage p + 1 from interval 4p - 1 on: group 1
     // loads it in M(2p - 1) (4p - 1), group 0 in M(2p) (4p).  Its first reads are group 0's C(2p + 1), interval
@@ -772,7 +673,6 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
     // The loads of stages it + NST - 2 and it + NST - 1 go to the slots of stages it - 2 and it - 1,
     // which every wave finished reading before the last barrier (lgkmcnt(0) ahead of it).  The MFMAs of
     // an output element run over the k-steps in the same order as in the other loops.
-    static_assert(C::QH == C::QL, "uniform loads per wave");
     u32x4 xa0[C::MT], xb0[C::NTL], xa1[C::MT], xb1[C::NTL], xa2[C::MT], xb2[C::NTL], xa3[C::MT], xb3[C::NTL];
     rd(smem, ao0, bo0, xa0, xb0);
     rd(smem, ao1, bo1, xa1, xb1);

@@ -1669,9 +1669,9 @@ int launch_gemm_skinny(const GemmArgs& g, hipStream_t st) {
 
 int launch_lm_head(const GemmArgs& g0, hipStream_t st) {
   // Up to 64 rows per pass.  The batch kernel takes whole 512-byte K chunks; a single row over more than
-  // three of them is faster on the skinny kernel, which has no barriers to pay for (measured above).
+  // six of them is faster on the skinny kernel, which has no barriers to pay for (measured above).
   const bool whole = g0.K > 0 && g0.K * 2 % LH_KB == 0;
-  const int lo = whole && g0.K * 2 <= 3 * LH_KB ? 0 : 1;
+  const int lo = whole && g0.K * 2 <= 6 * LH_KB ? 0 : 1;
   for (int m0 = 0, rows; m0 < g0.M; m0 += rows) {
     GemmArgs g = g0;
     const int left = g0.M - m0;

@@ -532,7 +532,7 @@ def test_lm_head_batches(V, H):
     for B in (1, 2, 15, 16, 17, 32, 33, 48, 49, 64, 65, 80, 128):
         out = ops.lm_head(x[:B].contiguous(), w)
         assert ((out.double() - ref[:B]).abs() <= bound[:B]).all(), B
-        # a single row over more than 768 k takes the skinny kernel: same sums, same bits
+        # a single row over more than 1536 k takes the skinny kernel: same sums, same bits
         assert torch.equal(out.view(torch.int32), full[:B].view(torch.int32)), B
 
 

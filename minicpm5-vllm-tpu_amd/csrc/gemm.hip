@@ -24,6 +24,7 @@
 #include <cstdlib>
 #include <type_traits>
 
+#include "gemm_stage.h"
 #include "kernels.h"
 #include "mk_common.h"
 
@@ -186,11 +187,7 @@ __device__ inline void epi_store(const GemmArgs& g, int m, int n, float v) {
   }
 }
 
-// Stage s of the LDS ring holds A rows [0, BM) then B rows [0, BN), BKB bytes of K each.  16-byte
-// chunk c of row r sits at slot c ^ swz(r), so the 16 lanes of a ds_read_b128 phase (16 consecutive
-// rows, same chunk) hit 16 distinct 4-bank groups.
-template <int BKB>
-__device__ inline int swz(int row) { return BKB == 64 ? (row >> 2) & 3 : (row >> 1) & 7; }
+// Stage s of the LDS ring holds A rows [0, BM) then B rows [0, BN), BKB bytes of K each, swizzled (swz).
 
 // Workgroup barrier for the LDS ring.  A bare s_barrier: __syncthreads() adds a fence that would also
 // drain the younger stages' async loads.  The empty asm statements keep the compiler from moving LDS
@@ -249,10 +246,10 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
     const int b = lw + C::NW * j;
     if (j < JA) {
       const int r = C::RPB * b + lane / C::CPR;
-      loff[j] = (uint32_t)min(m0 + r, g.M - 1) * (uint32_t)lda + 16u * ((lane % C::CPR) ^ swz<BKB>(r));
+      loff[j] = (uint32_t)min(m0 + r, g.M - 1) * (uint32_t)lda + 16u * stage_chunk<BKB>(lane, r);
     } else {
       const int r = C::RPB * (b - C::NA) + lane / C::CPR;
-      loff[j] = (uint32_t)min(n0 + r, g.N - 1) * (uint32_t)ldb + 16u * ((lane % C::CPR) ^ swz<BKB>(r));
+      loff[j] = (uint32_t)min(n0 + r, g.N - 1) * (uint32_t)ldb + 16u * stage_chunk<BKB>(lane, r);
     }
   }
   // Lean addressing: load j's rows are 16 NW j rows past load 0's (A) or load JA's (B), with the same
@@ -288,10 +285,12 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
     if (j < JA) copy16_to_lds(rA, voff(j), (uint32_t)kb, dst);
     else copy16_to_lds(rB, voff(j), (uint32_t)kb, dst);
   };
-  // A last stage of half the K bytes (LOOP 4): its other half would read past the row (unused), and past the
-  // last row out of the buffer, so the K offset goes where the range check sees it (out of range: zeros).
+  // A last stage of half the K bytes (LOOP 4): the lanes of its other half read nothing.  The rows of a lane's
+  // loads are multiples of 16 apart, so they share one swizzle; the K offset goes where the range check sees it.
   auto issue_half = [&](int j, int st, int kb) {
-    copy16_to_lds(j < JA ? rA : rB, voff(j) + (uint32_t)kb, smem + st * C::ST_BYTES + (lw + C::NW * j) * 1024);
+    static_assert(C::LOOP != 4 || (C::RPB * C::NW % 16 == 0 && C::BM % 16 == 0), "one swizzle per lane");
+    copy16_to_lds(j < JA ? rA : rB, half_stage_offset<BKB>(voff(j), lane, C::RPB * lw + lane / C::CPR, (uint32_t)kb),
+                  smem + st * C::ST_BYTES + (lw + C::NW * j) * 1024);
   };
   // wait until at most `n` stages of this wave's async loads are outstanding
   auto wait_stages = [&](auto nc) {

@@ -358,6 +358,30 @@ def test_gemm_ping_pong_stages(N, kb):
     assert (err <= 1e-4 * (af.double().abs() @ bf.double().abs().t())).all()
 
 
+@pytest.mark.parametrize("N", [1536, 2048, 2560])
+@pytest.mark.parametrize("K", [32, 96, 800])
+def test_gemm_operand_column_range(N, K):
+    """bf16 operands that are the last K columns of wider matrices (row stride K + 40, the last row ends with the
+    allocation), K bytes an odd multiple of 64: the ping-pong tiles' half stage stops at K, f32 bits equal to those
+    of contiguous copies."""
+    import ctypes
+
+    from minicpm5_mk import _lib, ops
+
+    dev = _dev()
+    g = torch.Generator().manual_seed(N + K)
+    M, ld = 8100, K + 40
+    print(f"[column range] {M}x{N}x{K}", flush=True)
+    a = torch.randn(M, ld, generator=g).to(BF16).to(dev)[:, 40:]
+    b = torch.randn(N, ld, generator=g).to(BF16).to(dev)[:, 40:]
+    out = torch.empty(M, N, dtype=torch.float32, device=dev)
+    ptr = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    _lib.check(_lib.load().mk_gemm(0, _lib.EPI["f32"], ptr(a), ld, ptr(b), ld, M, N, K, ptr(out), N, None, 0, None, None,
+                                   None, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "mk_gemm")
+    ref = ops.gemm(a.contiguous(), b.contiguous(), "f32")
+    assert torch.equal(out.view(torch.int32), ref.view(torch.int32))
+
+
 @pytest.mark.parametrize("epi", ["f32", "bf16", "res_f32add", "res_bf16add"])
 def test_gemm_wide_tile_rows_match(epi):
     """M = 8192, N = 2560 takes the 256x320 tile (one round of 256 CUs; 64x160 wave tiles, the epilogue

@@ -658,14 +658,12 @@ int launch_attn_hd(const AttnArgs& a, hipStream_t st, int stages) {
     const int items8 = a.B * a.n_kv * (a.S / QT);
     // the prefetch ranges shrunk to the whole 16-byte vectors inside them
     PrefetchRanges pf{};
-    bool any_pf = false;
     for (int r = 0; r < 4; ++r) {
       if (!a.pf.p[r] || a.pf.bytes[r] < 32) continue;
       const uintptr_t b0 = reinterpret_cast<uintptr_t>(a.pf.p[r]), e0 = b0 + a.pf.bytes[r];
       const uintptr_t b16 = (b0 + 15) & ~(uintptr_t)15, e16 = e0 & ~(uintptr_t)15;
       pf.p[r] = reinterpret_cast<const void*>(b16);
       pf.bytes[r] = e16 - b16;
-      any_pf = true;
     }
     auto go = [&](auto gw) {
       constexpr int GW = decltype(gw)::value;
@@ -678,9 +676,10 @@ int launch_attn_hd(const AttnArgs& a, hipStream_t st, int stages) {
         // one persistent workgroup per CU taking items from the queues, or, with no more items than CUs, one
         // workgroup per item (no queues); with prefetch ranges, the CUs left over get prefetch-only workgroups
         const int nwork = items < ncu ? items : ncu;
-        const int grid = any_pf ? ncu : nwork;
+        const PrefetchRanges fit = prefetch_fit(pf, ncu - nwork, HD, a.S);
+        const int grid = prefetch_any(fit) ? ncu : nwork;
         hipLaunchKernelGGL((attn_fwd_kernel<HD, true, GW>), dim3(grid), dim3(64 * GW), 0, st, a.qkv, a.cos, a.sin,
-                           a.krope, a.vt, a.out, a.B, a.S, a.n_q, a.n_kv, a.qscale, queue, pf, nwork,
+                           a.krope, a.vt, a.out, a.B, a.S, a.n_q, a.n_kv, a.qscale, queue, fit, nwork,
                            nwork == items ? 1 : 0, (uint32_t*)nullptr);
       }
     };

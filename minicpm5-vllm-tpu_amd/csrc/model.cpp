@@ -424,10 +424,11 @@ int launch_forward(const Fwd& f, hipStream_t st) {
     // The weights of this layer's gate/up and O projections, of the next layer's QKV and of this layer's down
     // projection, read into the memory-side cache by the attention launch's spare workgroups (a short prompt
     // leaves CUs idle there).  The layers' weights together exceed that cache, so otherwise each GEMM of a
-    // short prompt streams its weights cold, a full HBM round trip per K stage.  Ranges in order of what a cold
-    // start costs (us, warm / cold, at M = 256: gate/up 9.6 / 14.2, O 9.7 / 10.5, QKV 6.2 / 7.1, down 17.8 /
-    // 19.3).  Down is last, within kPrefetchBudget: with its 25 MB (64 MB in all) the 2B forward takes 5.60 ms at
-    // (1, 1024) and 3.95 at (1, 512), without it 5.88 and 4.15, with gate/up left out instead 5.68 and 3.97.
+    // short prompt streams its weights cold, a full HBM round trip per K stage.  The launch reads the ranges that
+    // its spare workgroups can read in its own time (prefetch_fit), in order of what a cold start costs (us,
+    // warm / cold, at M = 256: gate/up 9.6 / 14.2, O 9.7 / 10.5, QKV 6.2 / 7.1, down 17.8 / 19.3).  Down is last,
+    // within kPrefetchBudget: with its 25 MB (64 MB in all) the 2B forward takes 5.60 ms at (1, 1024) and 3.95 at
+    // (1, 512), without it 5.88 and 4.15, with gate/up left out instead 5.68 and 3.97.
     constexpr size_t kPrefetchBudget = (size_t)96 << 20;
     aa.pf.p[0] = pb + m.P.wgu + (size_t)l * 2 * I * H * e2;
     aa.pf.bytes[0] = (size_t)2 * I * H * e2;

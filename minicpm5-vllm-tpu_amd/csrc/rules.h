@@ -1,0 +1,40 @@
+// Launch rules that are plain arithmetic on sizes (no HIP types: the CPU tests compile this header too).
+#pragma once
+
+#include <stddef.h>
+
+namespace mk {
+
+// Byte ranges that otherwise idle workgroups of a launch read and drop (attn.hip): a hint that leaves the
+// data in the memory-side cache for the launches that follow.  No result depends on it.
+struct PrefetchRanges {
+  const void* p[4];
+  size_t bytes[4];   // 0: unused
+};
+
+// The ranges that `spare` workgroups can read while an attention launch over sequences of S tokens runs anyway;
+// the launch lasts until the last of them is done.  One workgroup reads 72 - 75 KB/us (8 of them took 111 us for
+// the 2B layer's 64 MB); 64 KB/us are counted, over 8 us and, at hd 128, 1.25 us per 64-key tile of the longest
+// q tile.  Ranges are taken whole or left out: a GEMM waits for the cold rest of its weights as for all of them
+// (2B (12, 128), us per forward: nothing read 7029, 55 of 64 MB 7255, all 6948).  Forwards, us, without a
+// prefetch / all ranges / this rule: 2B (31, 128) 12844 / 17265 / 12841, (6, 640) 13047 / 14489 / 12957,
+// (1, 1920) 8959 / 9957 / 9133, (20, 128) 10469 / 9920 / 9938, (8, 128) 5555 / 5213 / 5212; 1B (31, 128)
+// 5164 / 6748 / 5192, (12, 128) 3189 / 3075 / 3077, (1, 512) 2119 / 1893 / 1894.
+inline PrefetchRanges prefetch_fit(PrefetchRanges pf, int spare, int hd, int S) {
+  const double us = 8.0 + 1.25 * hd / 128 * (S / 64);
+  double left = spare * 64.0 * 1024 * us;
+  for (int r = 0; r < 4; ++r) {
+    if ((double)pf.bytes[r] > left) {
+      pf.p[r] = nullptr;
+      pf.bytes[r] = 0;
+    }
+    left -= (double)pf.bytes[r];
+  }
+  return pf;
+}
+
+inline bool prefetch_any(const PrefetchRanges& pf) {
+  return pf.bytes[0] || pf.bytes[1] || pf.bytes[2] || pf.bytes[3];
+}
+
+}  // namespace mk

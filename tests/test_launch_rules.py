@@ -1,0 +1,64 @@
+"""The launch rules of csrc/rules.h, compiled with the host compiler and checked on the CPU."""
+import ctypes
+import os
+import shutil
+import subprocess
+
+import pytest
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+CSRC = os.path.join(ROOT, "minicpm5-vllm-tpu_amd", "csrc")
+
+SRC = r"""
+#include "rules.h"
+extern "C" void fit(const size_t* in, size_t* out, int spare, int hd, int S) {
+  mk::PrefetchRanges pf{};
+  for (int r = 0; r < 4; ++r) pf.p[r] = in[r] ? in : nullptr, pf.bytes[r] = in[r];
+  const mk::PrefetchRanges f = mk::prefetch_fit(pf, spare, hd, S);
+  for (int r = 0; r < 4; ++r) out[r] = f.bytes[r] && !f.p[r] ? ~(size_t)0 : f.bytes[r];
+}
+"""
+
+
+@pytest.fixture(scope="module")
+def rules(tmp_path_factory):
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        pytest.skip("no host C++ compiler")
+    d = tmp_path_factory.mktemp("rules")
+    (d / "rules.cpp").write_text(SRC)
+    subprocess.run([cxx, "-std=c++17", "-O1", "-shared", "-fPIC", f"-I{CSRC}", str(d / "rules.cpp"), "-o",
+                    str(d / "rules.so")], check=True)
+    return ctypes.CDLL(str(d / "rules.so"))
+
+
+# bytes of a layer's gate/up, O, next QKV and down weights (W8A8 gate/up and QKV, bf16 O and down)
+WEIGHTS = {"1b": (14155776, 6291456, 3932160, 14155776), "2b": (25165824, 8388608, 5242880, 25165824)}
+
+
+def _fit(rules, ranges, spare, hd, S):
+    a, out = (ctypes.c_size_t * 4)(*ranges), (ctypes.c_size_t * 4)()
+    rules.fit(a, out, spare, hd, S)
+    return tuple(out)
+
+
+@pytest.mark.parametrize("arch", ["1b", "2b"])
+@pytest.mark.parametrize("hd", [96, 128])
+def test_prefetch_within_the_launch(rules, arch, hd):
+    """Whole ranges only, and never more than the spare workgroups read (at most 75 KB/us each) while the launch
+    runs (8 us and 1.25 us per key tile at hd 128): 8 spare workgroups beside 31 sequences of 128 tokens took
+    111 us for the 2B layer's 64 MB."""
+    w = WEIGHTS[arch]
+    for spare in (0, 1, 8, 16, 40, 64, 96, 128, 240):
+        for S in (64, 128, 1024, 1920, 3968):
+            got = _fit(rules, w, spare, hd, S)
+            assert all(g in (0, b) for g, b in zip(got, w))
+            assert sum(got) <= spare * 75 * 1024 * (8 + 1.25 * hd / 128 * (S // 64))
+
+
+def test_prefetch_takes_what_fits(rules):
+    w1, w2 = WEIGHTS["1b"], WEIGHTS["2b"]
+    assert _fit(rules, w2, 8, 128, 128) == (0, 0, 5242880, 0)
+    assert _fit(rules, w2, 128, 128, 128) == w2 and _fit(rules, w1, 240, 128, 128) == w1
+    assert _fit(rules, w2, 16, 128, 1920) == w2[:3] + (0,)
+    assert _fit(rules, (0, 0, 0, 0), 8, 128, 128) == (0, 0, 0, 0)

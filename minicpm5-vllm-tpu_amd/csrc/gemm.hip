@@ -1667,16 +1667,14 @@ int launch_gemm_skinny(const GemmArgs& g, hipStream_t st) {
 }
 
 int launch_lm_head(const GemmArgs& g0, hipStream_t st) {
-  // Up to 64 rows per pass.  The batch kernel takes whole 512-byte K chunks; a single row over more than
-  // six of them is faster on the skinny kernel, which has no barriers to pay for (measured above).
+  // Up to 64 rows per pass.  The batch kernel takes whole 512-byte K chunks.
   const bool whole = g0.K > 0 && g0.K * 2 % LH_KB == 0;
-  const int lo = whole && g0.K * 2 <= 6 * LH_KB ? 0 : 1;
   for (int m0 = 0, rows; m0 < g0.M; m0 += rows) {
     GemmArgs g = g0;
     const int left = g0.M - m0;
     g.A = static_cast<const uint16_t*>(g0.A) + (size_t)m0 * g0.lda;
     g.out = static_cast<float*>(g0.out) + (size_t)m0 * g0.ldo;
-    if (!whole || left <= lo) {
+    if (!whole || lm_head_skinny(left, g0.N, g0.K)) {
       rows = g.M = std::min(32, left);
       const int rc = launch_gemm_skinny(g, st);
       if (rc) return rc;

@@ -98,7 +98,7 @@ struct GemmArgs {
 int gemm_validate(const GemmArgs& g);
 int launch_gemm(const GemmArgs& g, hipStream_t st);
 
-// Skinny GEMM for M <= 32 rows (last-token layer, LM head): same math, weights streamed once; with
+// Skinny GEMM for M <= 32 rows (last-token layer, LM heads of few rows): same math, weights streamed once; with
 // g.ws, the K range is split over more waves (partials summed in a fixed order by a second kernel).
 int launch_gemm_skinny(const GemmArgs& g, hipStream_t st);
 // Logits (F32 epilogue, bf16 operands) of any number of rows, the weights read once per 64 of them.

@@ -37,4 +37,16 @@ inline bool prefetch_any(const PrefetchRanges& pf) {
   return pf.bytes[0] || pf.bytes[1] || pf.bytes[2] || pf.bytes[3];
 }
 
+// Whether a pass of the LM head over `rows` rows (V columns, K elements) takes the skinny kernel: no barriers to pay
+// for and 64 columns per workgroup, where the batch kernel's workgroups hold 128.  So it wins while few rows share
+// the weights and its workgroups all run in one round of 256 CUs (us, skinny then batch kernel: V = 8192, H = 1536,
+// 1 row 10.3, 13.5, 8 rows 11.9, 13.5, 16 rows 13.7, 13.6; H = 4096, 2 rows 27.8, 33.6, 16 rows 31.5, 33.7;
+// V = 16384, H = 2048, 2 rows 8 % apart), but not beyond (V = 20480: the batch kernel takes 0.77 times as long).
+// There it wins for one row over more than six chunks of K (V = 130560, H = 2048: 93.4, 96.5), and for two where the
+// batch kernel's workgroups fill whole rounds of three per CU or more (95.7, 98.6; V = 65536: 9 % slower).
+inline bool lm_head_skinny(int rows, int V, int K) {
+  if (V <= 64 * 256 && rows <= (8 + K / 384 < 16 ? 8 + K / 384 : 16)) return true;
+  return K > 1536 && (rows == 1 || (rows == 2 && V >= 3 * 128 * 256));
+}
+
 }  // namespace mk

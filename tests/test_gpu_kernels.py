@@ -539,10 +539,10 @@ def _pack_gu_scales(s_il, inter):
     return s_il.reshape(-1)[src].contiguous()
 
 
-@pytest.mark.parametrize("V,H", [(1000, 1536), (1000, 2048), (520, 256), (520, 1152)])
+@pytest.mark.parametrize("V,H", [(1000, 1536), (1000, 2048), (520, 256), (520, 1152), (16392, 256), (16400, 2048)])
 def test_lm_head_batches(V, H):
     """Batches at the edges of the LM head's 16-row groups and 64-row passes (H = 1152: no whole 256-element
-    chunks, the 32-row kernel): f32 sums of exact bf16 products, so each logit is within 32 eps sum|products|
+    chunks, the 32-row kernel; above V = 16384 the batch kernel takes fewer than 17 rows too): f32 sums of exact bf16 products, so each logit is within 32 eps sum|products|
     of the float64 one, and a row's bits do not depend on the batch."""
     from minicpm5_mk import ops
 
@@ -556,7 +556,7 @@ def test_lm_head_batches(V, H):
     for B in (1, 2, 15, 16, 17, 32, 33, 48, 49, 64, 65, 80, 128):
         out = ops.lm_head(x[:B].contiguous(), w)
         assert ((out.double() - ref[:B]).abs() <= bound[:B]).all(), B
-        # a single row over more than 1536 k takes the skinny kernel: same sums, same bits
+        # few rows, or one over more than 1536 k, take the skinny kernel: same sums, same bits
         assert torch.equal(out.view(torch.int32), full[:B].view(torch.int32)), B
 
 

@@ -17,6 +17,7 @@ extern "C" void fit(const size_t* in, size_t* out, int spare, int hd, int S) {
   const mk::PrefetchRanges f = mk::prefetch_fit(pf, spare, hd, S);
   for (int r = 0; r < 4; ++r) out[r] = f.bytes[r] && !f.p[r] ? ~(size_t)0 : f.bytes[r];
 }
+extern "C" int lm_head_skinny(int rows, int V, int K) { return mk::lm_head_skinny(rows, V, K); }
 """
 
 
@@ -62,3 +63,15 @@ def test_prefetch_takes_what_fits(rules):
     assert _fit(rules, w2, 128, 128, 128) == w2 and _fit(rules, w1, 240, 128, 128) == w1
     assert _fit(rules, w2, 16, 128, 1920) == w2[:3] + (0,)
     assert _fit(rules, (0, 0, 0, 0), 8, 128, 128) == (0, 0, 0, 0)
+
+
+@pytest.mark.parametrize("rows,V,K,skinny", [
+    (1, 1000, 256, True), (1, 8192, 1536, True), (2, 1000, 4096, True), (8, 8192, 1536, True), (8, 8192, 256, True),
+    (12, 4096, 1536, True), (16, 1000, 4096, True), (1, 16384, 1536, True),
+    (17, 1000, 4096, False), (16, 8192, 1536, False), (33, 1000, 1536, False), (1, 20480, 1536, False),
+    (2, 20480, 2048, False), (1, 130560, 1536, False), (1, 130560, 2048, True), (2, 130560, 2048, True),
+    (2, 65536, 2048, False), (3, 130560, 2048, False), (40, 130560, 1536, False)])
+def test_lm_head_kernel_choice(rules, rows, V, K, skinny):
+    """Few rows over a vocabulary whose 64-column workgroups run in one round, and one or two rows over long rows,
+    take the skinny kernel (measured faster there), the rest the batch kernel."""
+    assert bool(rules.lm_head_skinny(rows, V, K)) == skinny

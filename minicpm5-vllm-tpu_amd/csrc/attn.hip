@@ -647,14 +647,9 @@ int launch_attn_hd(const AttnArgs& a, hipStream_t st, int stages) {
         n = 0;
       return n > 0 ? n : 256;
     }();
-    // Workgroups of 8 waves (the kv head's 8 q heads share every K / V tile), or of 4 (twice the items, one wave
-    // per SIMD) while every one of those still has a CU to itself: a step of a lone wave is 5 - 25 % shorter,
-    // so the longest q tile finishes sooner (us, 8 then 4 waves: 64 items hd 128 31.3, 25.8, hd 96 23.2, 21.5;
-    // 128 items hd 128 51.9, 45.1, hd 96 39.5, 37.7), but a CU that takes a second item loses more than that
-    // ((4, 768), 192 items: hd 128 27.3, 33.6, hd 96 20.8, 27.9; (2, 1536): hd 96 32.6, 36.8).  One long
-    // sequence at hd 128 has few long tiles, and the second items are its short ones: there 4 waves still win
-    // up to three quarters of the CUs ((1, 3072) 73.6, 70.3; (1, 3584) 83.2, 85.4).  Static pairs when they
-    // fill the CUs in whole rounds (no queue atomics, fixed XCD placement), else the work queues.
+    // Workgroups of 8 waves (the kv head's 8 q heads share every K / V tile) or of 4 (attn_waves).  Static
+    // pairs when they fill the CUs in whole rounds (no queue atomics, fixed XCD placement), else the work
+    // queues.
     const int items8 = a.B * a.n_kv * (a.S / QT);
     // the prefetch ranges shrunk to the whole 16-byte vectors inside them
     PrefetchRanges pf{};
@@ -683,7 +678,7 @@ int launch_attn_hd(const AttnArgs& a, hipStream_t st, int stages) {
                            nwork == items ? 1 : 0, (uint32_t*)nullptr);
       }
     };
-    if (2 * items8 <= ncu || (HD == 128 && a.B == 1 && 4 * items8 <= 3 * ncu)) go(std::integral_constant<int, 4>{});
+    if (attn_waves(items8, ncu, HD, a.B, prefetch_any(pf)) == 4) go(std::integral_constant<int, 4>{});
     else go(std::integral_constant<int, G>{});
     MK_HIP_CHECK(hipGetLastError());
   }

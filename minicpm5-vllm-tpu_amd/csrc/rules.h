@@ -37,6 +37,23 @@ inline bool prefetch_any(const PrefetchRanges& pf) {
   return pf.bytes[0] || pf.bytes[1] || pf.bytes[2] || pf.bytes[3];
 }
 
+// Waves per attention workgroup: 8, or 4, which doubles the items (items8 of 8 waves) and leaves one wave per SIMD.
+// A lone wave's step is 5 - 25 % shorter, so the longest q tile finishes sooner while every item has a CU to itself
+// (us, 8 then 4 waves: 64 items hd 128 31.3, 25.8, hd 96 23.2, 21.5; 128 items hd 128 51.9, 45.1, hd 96 39.5, 37.7).
+// Beyond that some CUs take a second item, which mostly costs more than it gains ((4, 768), 192 items: hd 128 27.3,
+// 33.6, hd 96 20.8, 27.9; (2, 1536): hd 96 32.6, 36.8).  At hd 128 a batch of one or two long sequences has few long
+// tiles and the second items are its short ones: there 4 waves still win, with the K / V preparation, up to 15/16 of
+// the CUs for one sequence ((1, 3200) 80.1, 74.3; (1, 3584) 87.8, 84.5; (1, 3840) 94.0, 93.5; (1, 3968) 97.5, 98.5)
+// and below 3/4 for two ((2, 1216) 41.2, 39.4; (2, 1344) 44.5, 42.8; (2, 1536) 48.6, 49.9).  Inside a model the CUs that 8
+// waves leave free read the next weights, which is worth more from 3/4 of the CUs on for one sequence (2B forward:
+// (1, 3456) 13.96 ms, 14.40; (1, 3840) 15.3, 15.9) and for two (1B (2, 1280) 3.98, 4.67).
+inline int attn_waves(int items8, int ncu, int hd, int B, bool prefetch) {
+  if (2 * items8 <= ncu) return 4;
+  if (hd == 128 && B == 1 && 16 * items8 <= (prefetch ? 12 : 15) * ncu) return 4;
+  if (hd == 128 && B == 2 && 4 * items8 < 3 * ncu && !prefetch) return 4;
+  return 8;
+}
+
 // Whether a pass of the LM head over `rows` rows (V columns, K elements) takes the skinny kernel: no barriers to pay
 // for and 64 columns per workgroup, where the batch kernel's workgroups hold 128.  So it wins while few rows share
 // the weights and its workgroups all run in one round of 256 CUs (us, skinny then batch kernel: V = 8192, H = 1536,

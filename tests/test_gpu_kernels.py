@@ -44,7 +44,8 @@ def _attn_inputs(B, S, hd, n_q=16, n_kv=2):
 
 @pytest.mark.parametrize("B,S,hd,theta", [(1, 256, 64, 1e4), (2, 512, 96, 1e4), (1, 1024, 128, 5e6),
                                            (3, 128, 128, 5e6), (2, 384, 96, 1e4), (1, 640, 128, 5e6),
-                                           (1, 8192, 96, 1e4), (1, 8192, 128, 5e6), (3, 2048, 128, 5e6)])
+                                           (1, 8192, 96, 1e4), (1, 8192, 128, 5e6), (3, 2048, 128, 5e6),
+                                           (1, 3136, 128, 5e6)])
 def test_attention_vs_fp32(B, S, hd, theta):
     from minicpm5_mk import ops
     from minicpm5_mk.mk_weights import rope_tables
@@ -101,14 +102,16 @@ def test_attention_deterministic():
     assert torch.equal(a, b)
 
 
-@pytest.mark.parametrize("B,S,hd", [(2, 4096, 128), (4, 2048, 96), (3, 2048, 128), (4, 768, 96), (4, 768, 64)])
+@pytest.mark.parametrize("B,S,hd", [(2, 4096, 128), (4, 2048, 96), (3, 2048, 128), (4, 768, 96), (4, 768, 64),
+                                    (2, 2560, 128), (2, 3392, 128), (2, 1216, 128)])
 def test_attention_batch_invariant(B, S, hd):
     """Each sequence of a batch equals the same sequence run alone, bit for bit.  (2, 4096) and
     (4, 2048) launch 256 tile pairs (B * 2 kv heads * S / 64) and take the static pair mapping;
     (3, 2048) launches 384 items on 256 persistent workgroups, so workgroups take several items and
     drain the other kv head's queue; the single-sequence runs have no more items than CUs and take the
     direct mapping (workgroup i computes item i, no queue).  (4, 768) launches 192 items of 8 waves, its
-    single sequences items of 4 waves."""
+    single sequences items of 4 waves.  The single sequences of (2, 2560) and (2, 3392), and the batch
+    (2, 1216), launch more 4-wave items than there are CUs and take them from the queues."""
     from minicpm5_mk import ops
     from minicpm5_mk.mk_weights import rope_tables
 

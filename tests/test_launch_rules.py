@@ -17,6 +17,9 @@ extern "C" void fit(const size_t* in, size_t* out, int spare, int hd, int S) {
   const mk::PrefetchRanges f = mk::prefetch_fit(pf, spare, hd, S);
   for (int r = 0; r < 4; ++r) out[r] = f.bytes[r] && !f.p[r] ? ~(size_t)0 : f.bytes[r];
 }
+extern "C" int attn_waves(int items8, int ncu, int hd, int B, int prefetch) {
+  return mk::attn_waves(items8, ncu, hd, B, prefetch);
+}
 extern "C" int lm_head_skinny(int rows, int V, int K) { return mk::lm_head_skinny(rows, V, K); }
 """
 
@@ -75,3 +78,14 @@ def test_lm_head_kernel_choice(rules, rows, V, K, skinny):
     """Few rows over a vocabulary whose 64-column workgroups run in one round, and one or two rows over long rows,
     take the skinny kernel (measured faster there), the rest the batch kernel."""
     assert bool(rules.lm_head_skinny(rows, V, K)) == skinny
+
+
+@pytest.mark.parametrize("B,S,hd,prefetch,waves", [
+    (1, 2048, 64, False, 4), (16, 128, 96, True, 4), (1, 3136, 128, False, 4), (1, 3456, 128, False, 4),
+    (1, 3840, 128, False, 4), (2, 1088, 128, False, 4), (2, 1472, 128, False, 4), (1, 3072, 128, True, 4),
+    (1, 3904, 128, False, 8), (1, 3136, 128, True, 8), (1, 3840, 128, True, 8), (2, 1536, 128, False, 8),
+    (2, 1088, 128, True, 8), (1, 2112, 96, False, 8), (2, 1088, 64, False, 8), (3, 704, 128, False, 8),
+    (4, 768, 128, False, 8), (1, 4096, 128, False, 8), (1, 8192, 128, True, 8)])
+def test_attention_waves(rules, B, S, hd, prefetch, waves):
+    """Waves per attention workgroup on 256 CUs (2 kv heads, 32-token q tiles)."""
+    assert rules.attn_waves(B * 2 * (S // 32), 256, hd, B, int(prefetch)) == waves

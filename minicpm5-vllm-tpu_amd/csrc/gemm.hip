@@ -84,8 +84,6 @@ struct GemmCfg {
   // they are used instead of being held through the main loop (held, they spilled into the loop).
   static constexpr bool LEAN = LOOP == 4 && 16 * MT * NTL + 12 * (MT + NTL) > 190;
 };
-// 256x256 block, 128x128 per wave (accumulators in AGPRs), one workgroup per CU
-using CfgL = GemmCfg<256, 256, 2, 2, 3, 1, 0>;
 // 256x128 block, 128x64 per wave, two workgroups per CU
 using CfgM = GemmCfg<256, 128, 2, 2, 3, 2>;
 // 128x128 block, 64x64 per wave, three workgroups per CU
@@ -1368,12 +1366,12 @@ int choose_cfg(const GemmArgs& g) {
   // 5, 8, 9, 10: waves without whole [gate | up] blocks; 12: built for SiLU alone; 6, 9 - 13: whole lines
   auto ok = [&](int id) {
     if (id == 8) return wide320;
-    if (silu) return (id >= 1 && id <= 7 && id != 5 && id != 6) || (line && id == 12);
-    return id >= 1 && id <= 13 && id != 12 && (line || !(id == 6 || id >= 9));
+    if (silu) return (id >= 2 && id <= 7 && id != 5 && id != 6) || (line && id == 12);
+    return id >= 2 && id <= 13 && id != 12 && (line || !(id == 6 || id >= 9));
   };
   if (ok(g.cfg)) return g.cfg;
   static const int forced = [] {
-    const char* e = std::getenv("MK_GEMM_CFG");   // tuning override: 1 .. 13
+    const char* e = std::getenv("MK_GEMM_CFG");   // tuning override: 2 .. 13
     return e ? std::atoi(e) : 0;
   }();
   if (ok(forced)) return forced;
@@ -1404,8 +1402,8 @@ int choose_cfg(const GemmArgs& g) {
     if (silu && fits(128, 128)) return 3;
   }
   struct Opt { int id, bm, bn; double eff; };
-  const Opt opts[7] = {{4, 256, 256, silu ? 1.10 : 1.33}, {2, 256, 128, 1.0}, {1, 256, 256, 0.9},
-                       {3, 128, 128, 0.85}, {5, 256, 192, 1.25}, {8, 256, 320, 1.14}, {12, 192, 128, 1.0}};
+  const Opt opts[6] = {{4, 256, 256, silu ? 1.10 : 1.33}, {2, 256, 128, 1.0}, {3, 128, 128, 0.85},
+                       {5, 256, 192, 1.25},               {8, 256, 320, 1.14}, {12, 192, 128, 1.0}};
   int best = 2;
   double bt = 1e300;
   for (const Opt& o : opts) {
@@ -1466,7 +1464,6 @@ template <GemmIn IN, Epi EPI>
 void launch_t(const GemmArgs& g, hipStream_t st) {
   constexpr bool silu = EPI == Epi::DQ_SILU || EPI == Epi::DQ_SILU_F32A || EPI == Epi::SILU_BF16;
   switch (choose_cfg(g)) {
-    case 1: launch_c<CfgL, IN, EPI>(g, st); break;
     case 3: launch_c<CfgS, IN, EPI>(g, st); break;
     case 4: launch_c<CfgX, IN, EPI>(g, st); break;
     case 5:   // 96-column waves cannot hold whole [gate | up] blocks: SiLU epilogues take the 256x128 tile

@@ -76,10 +76,11 @@ struct GemmArgs {
   const float* rs;            // per-row scale (tokens)
   const float* cs;            // per-column scale (output channels)
   const float* aux;           // DQ_SILU_F32A: per-intermediate-channel factor
-  int cfg;                    // tile configuration: 0 auto, 1 256x256 (4 waves), 2 256x128, 3 128x128,
-                              // 4 256x256 (8 waves), 5 256x192 (8 waves; not for the SiLU epilogues),
-                              // 6 128x128 and 7 64x128 with 8-stage rings (short, long-K problems),
-                              // 8 256x320 (8 waves; not for the SiLU epilogues)
+  int cfg;                    // tile configuration: 0 auto, else (8 waves and one workgroup per CU, ping-pong:) 4
+                              // 256x256, 5 256x192, 8 256x320; (4 waves, 2 - 3 workgroups per CU:) 2 256x128,
+                              // 3 128x128, 12 192x128, 13 128x128; (short problems:) 7 64x128 in an 8-stage ring,
+                              // and with loader waves 6 128x128, 11 64x128, 9 64x64, 10 32x64.  A configuration
+                              // that is not built for the operands, epilogue or K counts as 0.
   int gm;                     // tile-order group height (rows of tiles); 0 = chosen by the launcher
   void* ws;                   // skinny GEMM: optional f32 workspace for split-K partials (null = no split)
   size_t ws_bytes;

@@ -407,7 +407,7 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
         for (int j = 0; j < Q; ++j) issue1(j, s0, s0 * BKB);
       }
     if (C::LOOP == 3) wait_newer(std::integral_constant<int, PRE - 2>{}, nk - 2);
-    else if (nk >= PRE) wait_stages(std::integral_constant<int, C::LOOP == 2 || C::LOOP == 3 ? PRE - 2 : PRE - 1>{});
+    else if (nk >= PRE) wait_stages(std::integral_constant<int, C::LOOP == 2 ? PRE - 2 : PRE - 1>{});
     else wait_stages(W0{});
   }
   lds_barrier();
@@ -1346,79 +1346,19 @@ __global__ __launch_bounds__(256) void skinny_reduce_kernel(GemmArgs g, int spli
   epi_store<EPI>(g, m, n, v);
 }
 
-// Tile configuration for a problem.  The busiest CU runs ceil(tiles / 256) tiles (the order spreads
-// them evenly), so the estimate is ceil(tiles / 256) * tile area / relative throughput, the throughputs
-// measured on MI355X at the model's shapes (random data): the 8-wave ping-pong 256x256 tile is fastest
-// per tile, except for the SiLU epilogue, whose VALU work is hidden better by two co-resident
-// 256x128 workgroups.  The 256x320 tile's 1.14: the QKV shape M = 8192, N = 2560, K = 1536 (dequantising
-// epilogue, no routing) takes 40.9 us on it, 48.6 us on 256x192 tiles (1.75 rounds) and 52.3 us on
-// 256x256 ones (1.25 rounds); with 128-byte stages 37.5 against 39.5 us, and 41.9 on 256x192.  The SiLU 256x256
-// tile's 1.10 (1.15 fits its own times, 125 us for the 1B gate/up at M = 8192 against 130 on 256x128 pairs):
-// inside the model the pairs take 127 us there against 130, and the attention next to them 231 against 240.
+// The tile of a problem: the caller's or the tuning override's if it is built and K is whole lines where its stages
+// are, else by size.
 int choose_cfg(const GemmArgs& g) {
   const bool silu = g.epi == Epi::DQ_SILU || g.epi == Epi::DQ_SILU_F32A || g.epi == Epi::SILU_BF16;
-  // 5 and 8 (96- and 160-column waves) cannot hold whole [gate | up] blocks
-  // fp8 stages are one wide k-step, held in four operand sets: with the 256x320 tile's 160 accumulators
-  // they exceed a wave's 256 registers
-  const bool wide320 = !silu && g.in != GemmIn::F8;
   const int kb = g.K * (g.in == GemmIn::BF16 ? 2 : 1);   // bytes
-  const bool line = kb % 128 == 0;                        // whole 128-byte stages
-  // 5, 8, 9, 10: waves without whole [gate | up] blocks; 12: built for SiLU alone; 6, 9 - 13: whole lines
-  auto ok = [&](int id) {
-    if (id == 8) return wide320;
-    if (silu) return (id >= 2 && id <= 7 && id != 5 && id != 6) || (line && id == 12);
-    return id >= 2 && id <= 13 && id != 12 && (line || !(id == 6 || id >= 9));
-  };
+  auto ok = [&](int id) { return gemm_tile_built(id, silu, g.in) && (kb % 128 == 0 || !(id == 6 || id >= 9)); };
   if (ok(g.cfg)) return g.cfg;
   static const int forced = [] {
     const char* e = std::getenv("MK_GEMM_CFG");   // tuning override: 2 .. 13
     return e ? std::atoi(e) : 0;
   }();
   if (ok(forced)) return forced;
-  // Few tiles (short prompts): the smallest tile whose tiling fits one round of 256 CUs, on whole-line stages.
-  // Measured on MI355X over M = 40 .. 3072 at the model's shapes, us warm / with cold weights, against the next
-  // larger choice:
-  //   32x64   1B down M = 256  17.8 / 19.3 (64x64 17.8 / 23.2), 2B down M = 128  21.9 / 25.0 (22.1 / 31.3)
-  //   64x64   1B down M = 512  19.1 / 23.4 (64x128 25.4 / 33.5), 1B QKV M = 384  6.5 / 7.1 (8.1 / 9.7)
-  //   64x128  1B down M = 1024  27.3 / 32.9 (64x128 with 64-byte stages 30.5 / 43.6); K loops of 32 or more
-  //           lines only: at 12 (int8, K = 1536) the 64-byte stages start sooner, 7.5 against 8.3 at M = 512
-  //   128x128 1B down M = 2048  40.4 / 43.6 (64-byte stages 44.3 / 55.0), likewise for 32 or more lines
-  // The SiLU epilogues need 64-column waves: 64x128 with 64-byte stages (1B gate/up M = 128  6.9 / 11.8 against
-  // 7.9 / 9.9 on whole lines), then 128x128 with three workgroups per CU (M = 256  9.6 / 14.2 against
-  // 13.7 / 17.8 on 256x128 tiles, M = 384  11.0 / 14.6 against 14.8 / 17.9).
-  {
-    const int lines = kb / 128;
-    auto fits = [&](int bm, int bn) { return (long)((g.M + bm - 1) / bm) * ((g.N + bn - 1) / bn) <= 256; };
-    if (!silu && line) {
-      if (fits(32, 64)) return 10;
-      if (fits(64, 64)) return 9;
-      if (lines >= 32 && fits(64, 128)) return 11;
-    }
-    if (kb >= 1024 && fits(64, 128)) return 7;
-    if (!silu && line && lines >= 32 && fits(128, 128)) return 6;
-    // up to two 128x128 workgroups per CU: 1B down at M = 4096 72.3 -> 60.4 us (before: one 256x128 tile per CU),
-    // O at M = 3072 34.5 -> 29.5, QKV at M = 2500 19.4 -> 18.0, 2B down at M = 4096 103 -> 96.9 (256x256 109)
-    if (!silu && line && !fits(128, 128) && (long)((g.M + 127) / 128) * ((g.N + 127) / 128) <= 512) return 13;
-    if (silu && fits(128, 128)) return 3;
-  }
-  struct Opt { int id, bm, bn; double eff; };
-  const Opt opts[6] = {{4, 256, 256, silu ? 1.10 : 1.33}, {2, 256, 128, 1.0}, {3, 128, 128, 0.85},
-                       {5, 256, 192, 1.25},               {8, 256, 320, 1.14}, {12, 192, 128, 1.0}};
-  int best = 2;
-  double bt = 1e300;
-  for (const Opt& o : opts) {
-    if ((silu && (o.id == 3 || o.id == 5)) || (!wide320 && o.id == 8)) continue;   // 3: never faster; 5, 8: no SiLU
-    // 192x128 pairs fill rounds the larger tiles leave half empty: 2B gate/up at M = 1536 52.0 -> 43.9 us, at
-    // M = 3072 88.4 -> 82.6, 1B gate/up at M = 6000 103 -> 96.7
-    if (o.id == 12 && !(silu && line)) continue;
-    const double tiles = (double)((g.M + o.bm - 1) / o.bm) * ((g.N + o.bn - 1) / o.bn);
-    const double t = std::ceil(tiles / 256.0) * o.bm * o.bn / o.eff;
-    if (t < bt * 0.999) {
-      bt = t;
-      best = o.id;
-    }
-  }
-  return best;
+  return gemm_tile(silu, g.in, g.M, g.N, kb);
 }
 
 // Tile-order group height (rows of tiles per group; the kernel walks each group column by column and
@@ -1460,41 +1400,37 @@ void launch_c(const GemmArgs& g0, hipStream_t st) {
                      0, st, g);
 }
 
+template <int ID>
+struct TileOf;
+template <> struct TileOf<2> { using C = CfgM; };
+template <> struct TileOf<3> { using C = CfgS; };
+template <> struct TileOf<4> { using C = CfgX; };
+template <> struct TileOf<5> { using C = CfgN; };
+template <> struct TileOf<6> { using C = CfgD; };
+template <> struct TileOf<7> { using C = CfgE; };
+template <> struct TileOf<8> { using C = CfgW; };
+template <> struct TileOf<9> { using C = CfgF; };
+template <> struct TileOf<10> { using C = CfgG; };
+template <> struct TileOf<11> { using C = CfgH; };
+template <> struct TileOf<12> { using C = CfgP; };
+template <> struct TileOf<13> { using C = CfgQ; };
+
 template <GemmIn IN, Epi EPI>
-void launch_t(const GemmArgs& g, hipStream_t st) {
+int launch_t(const GemmArgs& g, hipStream_t st) {
   constexpr bool silu = EPI == Epi::DQ_SILU || EPI == Epi::DQ_SILU_F32A || EPI == Epi::SILU_BF16;
-  switch (choose_cfg(g)) {
-    case 3: launch_c<CfgS, IN, EPI>(g, st); break;
-    case 4: launch_c<CfgX, IN, EPI>(g, st); break;
-    case 5:   // 96-column waves cannot hold whole [gate | up] blocks: SiLU epilogues take the 256x128 tile
-      if constexpr (!silu) launch_c<CfgN, IN, EPI>(g, st);
-      else launch_c<CfgM, IN, EPI>(g, st);
-      break;
-    case 8:   // 160-column waves: likewise
-      if constexpr (!silu && IN != GemmIn::F8) launch_c<CfgW, IN, EPI>(g, st);
-      else launch_c<CfgM, IN, EPI>(g, st);
-      break;
-    case 6:
-      if constexpr (!silu) launch_c<CfgD, IN, EPI>(g, st);
-      break;
-    case 7: launch_c<CfgE, IN, EPI>(g, st); break;
-    case 9:
-      if constexpr (!silu) launch_c<CfgF, IN, EPI>(g, st);
-      break;
-    case 10:
-      if constexpr (!silu) launch_c<CfgG, IN, EPI>(g, st);
-      break;
-    case 11:
-      if constexpr (!silu) launch_c<CfgH, IN, EPI>(g, st);
-      break;
-    case 12:
-      if constexpr (silu) launch_c<CfgP, IN, EPI>(g, st);
-      break;
-    case 13:
-      if constexpr (!silu) launch_c<CfgQ, IN, EPI>(g, st);
-      break;
-    default: launch_c<CfgM, IN, EPI>(g, st); break;
+  const int id = choose_cfg(g);
+#define MK_TILE(ID)                                          \
+  if constexpr (gemm_tile_built(ID, silu, IN)) {             \
+    if (id == ID) {                                          \
+      launch_c<typename TileOf<ID>::C, IN, EPI>(g, st);      \
+      return MK_OK;                                          \
+    }                                                        \
   }
+  MK_TILE(2) MK_TILE(3) MK_TILE(4) MK_TILE(5) MK_TILE(6) MK_TILE(7)
+  MK_TILE(8) MK_TILE(9) MK_TILE(10) MK_TILE(11) MK_TILE(12) MK_TILE(13)
+#undef MK_TILE
+  set_error("gemm: the chosen tile is not built for this epilogue and operand type");
+  return MK_EUNSUPPORTED;
 }
 
 // K splits of a skinny GEMM: enough waves to keep HBM busy (~2048 over the chip), each split at least
@@ -1555,10 +1491,13 @@ int launch_e(const GemmArgs& g, hipStream_t st, bool skinny) {
         set_error("gemm: the SiLU epilogues have no skinny variant");
         return MK_EUNSUPPORTED;
       }
-      launch_t<IN, E>(g, st);
+      const int rc = launch_t<IN, E>(g, st);
+      if (rc) return rc;
+    } else if (skinny) {
+      launch_skinny_t<IN, E>(g, st);
     } else {
-      if (skinny) launch_skinny_t<IN, E>(g, st);
-      else launch_t<IN, E>(g, st);
+      const int rc = launch_t<IN, E>(g, st);
+      if (rc) return rc;
     }
     MK_HIP_CHECK(hipGetLastError());
     return MK_OK;

@@ -49,7 +49,6 @@ int launch_last_attn(const LastAttnArgs& a, hipStream_t st);
 
 // ------------------------------------------------------------------------------ GEMM
 // C(M, N) = A(M, K) * B(N, K)^T with A and B K-contiguous (row stride lda / ldb elements).
-enum class GemmIn { I8, BF16, F8 };   // F8: OCP e4m3 operands, f32 accumulation
 enum class Epi {
   DQ_BF16,        // out = bf16((acc * rs[m]) * cs[n])                      (fused_qkv)
   DQ_SILU,        // g/u interleaved by 32 columns: h = silu(g) * u, g,u = (acc * rs[m]) * cs[n]

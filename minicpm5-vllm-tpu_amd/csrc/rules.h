@@ -5,6 +5,74 @@
 
 namespace mk {
 
+enum class GemmIn { I8, BF16, F8 };   // operands of a GEMM; F8: OCP e4m3 operands, f32 accumulation
+
+// Whether GEMM tile `id` (GemmArgs::cfg) is built.  The SiLU epilogues need waves that hold whole 64-column
+// [gate | up] blocks, which 5, 8, 9 and 10 have not; 6, 11 and 13 are never the faster choice for them, 12 only
+// for them.  fp8 stages are one wide k-step held in four operand sets: with the 256x320 tile's 160 accumulators
+// they exceed a wave's 256 registers.
+constexpr bool gemm_tile_built(int id, bool silu, GemmIn in) {
+  return silu ? id == 2 || id == 3 || id == 4 || id == 7 || id == 12
+              : id >= 2 && id <= 13 && id != 12 && !(id == 8 && in == GemmIn::F8);
+}
+
+// Tile configuration for a problem: M x N outputs, kb bytes of K.  The busiest CU runs ceil(tiles / 256) tiles (the
+// order spreads them evenly), so the estimate is ceil(tiles / 256) * tile area / relative throughput, the throughputs
+// measured on MI355X at the model's shapes (random data): the 8-wave ping-pong 256x256 tile is fastest per tile,
+// except for the SiLU epilogue, whose VALU work is hidden better by two co-resident 256x128 workgroups.  The 256x320
+// tile's 1.14: the QKV shape M = 8192, N = 2560, K = 1536 (dequantising epilogue, no routing) takes 40.9 us on it,
+// 48.6 us on 256x192 tiles (1.75 rounds) and 52.3 us on 256x256 ones (1.25 rounds); with 128-byte stages 37.5 against
+// 39.5 us, and 41.9 on 256x192.  The SiLU 256x256 tile's 1.10 (1.15 fits its own times, 125 us for the 1B gate/up at
+// M = 8192 against 130 on 256x128 pairs): inside the model the pairs take 127 us there against 130, and the attention
+// next to them 231 against 240.
+inline int gemm_tile(bool silu, GemmIn in, int M, int N, int kb) {
+  const bool line = kb % 128 == 0;   // whole 128-byte stages
+  const int lines = kb / 128;
+  auto tiles = [&](int bm, int bn) { return (long)((M + bm - 1) / bm) * ((N + bn - 1) / bn); };
+  auto fits = [&](int bm, int bn) { return tiles(bm, bn) <= 256; };
+  // Few tiles (short prompts): the smallest tile whose tiling fits one round of 256 CUs, on whole-line stages.
+  // Measured on MI355X over M = 40 .. 3072 at the model's shapes, us warm / with cold weights, against the next
+  // larger choice:
+  //   32x64   1B down M = 256  17.8 / 19.3 (64x64 17.8 / 23.2), 2B down M = 128  21.9 / 25.0 (22.1 / 31.3)
+  //   64x64   1B down M = 512  19.1 / 23.4 (64x128 25.4 / 33.5), 1B QKV M = 384  6.5 / 7.1 (8.1 / 9.7)
+  //   64x128  1B down M = 1024  27.3 / 32.9 (64x128 with 64-byte stages 30.5 / 43.6); K loops of 32 or more
+  //           lines only: at 12 (int8, K = 1536) the 64-byte stages start sooner, 7.5 against 8.3 at M = 512
+  //   128x128 1B down M = 2048  40.4 / 43.6 (64-byte stages 44.3 / 55.0), likewise for 32 or more lines
+  // The SiLU epilogues need 64-column waves: 64x128 with 64-byte stages (1B gate/up M = 128  6.9 / 11.8 against
+  // 7.9 / 9.9 on whole lines), then 128x128 with three workgroups per CU (M = 256  9.6 / 14.2 against
+  // 13.7 / 17.8 on 256x128 tiles, M = 384  11.0 / 14.6 against 14.8 / 17.9).
+  if (!silu && line) {
+    if (fits(32, 64)) return 10;
+    if (fits(64, 64)) return 9;
+    if (lines >= 32 && fits(64, 128)) return 11;
+  }
+  if (kb >= 1024 && fits(64, 128)) return 7;
+  if (!silu && line && lines >= 32 && fits(128, 128)) return 6;
+  // up to two 128x128 workgroups per CU: 1B down at M = 4096 72.3 -> 60.4 us (before: one 256x128 tile per CU),
+  // O at M = 3072 34.5 -> 29.5, QKV at M = 2500 19.4 -> 18.0, 2B down at M = 4096 103 -> 96.9 (256x256 109)
+  if (!silu && line && !fits(128, 128) && tiles(128, 128) <= 512) return 13;
+  if (silu && fits(128, 128)) return 3;
+  struct Opt { int id, bm, bn; double eff; };
+  const Opt opts[6] = {{4, 256, 256, silu ? 1.10 : 1.33}, {2, 256, 128, 1.0}, {3, 128, 128, 0.85},
+                       {5, 256, 192, 1.25},               {8, 256, 320, 1.14}, {12, 192, 128, 1.0}};
+  int best = 2;
+  double bt = 1e300;
+  for (const Opt& o : opts) {
+    if (!gemm_tile_built(o.id, silu, in)) continue;
+    if (silu && o.id == 3) continue;   // the problems it is the faster SiLU tile for are above
+    // 192x128 pairs fill rounds the larger tiles leave half empty: 2B gate/up at M = 1536 52.0 -> 43.9 us, at
+    // M = 3072 88.4 -> 82.6, 1B gate/up at M = 6000 103 -> 96.7
+    if (o.id == 12 && !line) continue;
+    const long rounds = (tiles(o.bm, o.bn) + 255) / 256;
+    const double t = (double)rounds * o.bm * o.bn / o.eff;
+    if (t < bt * 0.999) {
+      bt = t;
+      best = o.id;
+    }
+  }
+  return best;
+}
+
 // Byte ranges that otherwise idle workgroups of a launch read and drop (attn.hip): a hint that leaves the
 // data in the memory-side cache for the launches that follow.  No result depends on it.
 struct PrefetchRanges {

@@ -17,6 +17,10 @@ extern "C" void fit(const size_t* in, size_t* out, int spare, int hd, int S) {
   const mk::PrefetchRanges f = mk::prefetch_fit(pf, spare, hd, S);
   for (int r = 0; r < 4; ++r) out[r] = f.bytes[r] && !f.p[r] ? ~(size_t)0 : f.bytes[r];
 }
+extern "C" int gemm_tile(int silu, int in, int M, int N, int kb) {
+  return mk::gemm_tile(silu, (mk::GemmIn)in, M, N, kb);
+}
+extern "C" int gemm_tile_built(int id, int silu, int in) { return mk::gemm_tile_built(id, silu, (mk::GemmIn)in); }
 extern "C" int attn_waves(int items8, int ncu, int hd, int B, int prefetch) {
   return mk::attn_waves(items8, ncu, hd, B, prefetch);
 }
@@ -89,3 +93,21 @@ def test_lm_head_kernel_choice(rules, rows, V, K, skinny):
 def test_attention_waves(rules, B, S, hd, prefetch, waves):
     """Waves per attention workgroup on 256 CUs (2 kv heads, 32-token q tiles)."""
     assert rules.attn_waves(B * 2 * (S // 32), 256, hd, B, int(prefetch)) == waves
+
+
+I8, BF16, F8 = 0, 1, 2      # GemmIn
+
+
+def test_gemm_tile_is_built(rules):
+    """The dispatch rule picks a tile that is built for the operands and epilogue, and one of whole-line stages only
+    for K of whole lines, over sizes from one row to 70000."""
+    sizes = [1, 2, 31, 33, 63, 64, 65, 127, 129, 256, 257, 511, 700, 1000, 1537, 2048, 3000, 4097, 6000, 8192, 10923,
+             16384, 30000, 70000]
+    for silu in (0, 1):
+        for in_type in (I8, BF16, F8):
+            for M in sizes:
+                for N in (64, 128, 512, 1536, 1920, 2048, 2560, 4096, 9216, 12288, 40000):
+                    for kb in (64, 128, 192, 448, 960, 1024, 1088, 1536, 2048, 4096, 4160, 9216, 12288):
+                        t = rules.gemm_tile(silu, in_type, M, N, kb)
+                        assert rules.gemm_tile_built(t, silu, in_type), (silu, in_type, M, N, kb, t)
+                        assert kb % 128 == 0 or not (t == 6 or t >= 9), (silu, in_type, M, N, kb, t)

@@ -476,15 +476,23 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
     // quarter of the A rows (by column tile) and one of the BN / 64 parts of the B rows (by row tile), the
     // neighbours the rest.
     const bool pfw = w < 2;
-    uint32_t pfo;
-    {
-      const int tm = m0 / BM, tn = n0 / BN;
-      const uint32_t ra = (uint32_t)min(m0 + 64 * (tn % (BM / 64)) + lane, g.M - 1) * (uint32_t)lda;
-      const uint32_t rb = (uint32_t)min(n0 + 64 * (tm % (BN / 64)) + lane, g.N - 1) * (uint32_t)ldb;
-      pfo = w == 0 ? ra : rb;
-    }
+    const int pm = m0 + 64 * (n0 / BN % (BM / 64)), pn = n0 + 64 * (m0 / BM % (BN / 64));   // the first row touched
+    auto pf_row = [&](int l) {
+      return w == 0 ? (uint32_t)min(pm + l, g.M - 1) * (uint32_t)lda : (uint32_t)min(pn + l, g.N - 1) * (uint32_t)ldb;
+    };
+    const uint32_t pfo = LEAN ? 0 : pf_row(lane);
     auto prefetch = [&](int p) {
-      if (pfw && p < nk) copy4_to_lds(w == 0 ? rA : rB, pfo, (uint32_t)(p * BKB), smem + C::NST * C::ST_BYTES + w * 256);
+      if (!pfw || p >= nk) return;
+      uint32_t o = pfo;
+      if constexpr (LEAN) {
+        // lean addressing: from the lane number, at each use.  Held, the offset was spilled in the fp8 256x256
+        // SiLU instance, and its reload, behind the stage's loads, waited for all of them: 2B gate/up at
+        // M = 4096 114 us, now 99, at M = 8192 204, now 190.
+        uint32_t ones = ~0u;
+        asm volatile("" : "+s"(ones));
+        o = pf_row((int)__builtin_amdgcn_mbcnt_hi(ones, __builtin_amdgcn_mbcnt_lo(ones, 0)));
+      }
+      copy4_to_lds(w == 0 ? rA : rB, o, (uint32_t)(p * BKB), smem + C::NST * C::ST_BYTES + w * 256);
     };
     // group 0's wait for its loads: the prefetch issued after them may be outstanding
     auto wait_loads = [&](int p) {

@@ -10,6 +10,8 @@ its GPU code:
 * packed FP32 arithmetic: the sources are compiled with the packed-fp32-ops target feature off, so no
   such instruction is generated and none is written by hand.
 
+A third check keeps register spills out of the tiled GEMM's K loops.
+
 Skipped when the library has not been built or the ROCm tools are missing.
 """
 import os
@@ -24,6 +26,7 @@ ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 LIB = os.path.join(ROOT, "minicpm5-vllm-tpu_amd", "minicpm5_mk", "libmk.so")
 OBJDUMP = "/opt/rocm/llvm/bin/llvm-objdump"
 
+FUNCTION = re.compile(r"^[0-9a-f]+ <(\S+)>:")
 SCALAR_WRITES = re.compile(r"\bs_(store|buffer_store|scratch_store|atomic|buffer_atomic|dcache_wb|dcache_discard)\w*")
 PACKED_F32 = re.compile(r"\bv_pk_(add|mul|fma)_f32\b")
 
@@ -55,4 +58,27 @@ def test_device_code_rules():
         hits += sorted(set(m.group(0) for m in PACKED_F32.finditer(text)))
         if hits:
             bad[f] = hits
+    assert not bad, bad
+
+
+def test_gemm_loops_do_not_spill():
+    """No scratch access between the first and the last matrix instruction of a tiled GEMM instance: a reload there
+    waits for every async load issued before it, so one spilled offset drained a whole stage per iteration."""
+    bad, seen = {}, 0
+    for text in _disassembly().values():
+        name, mfmas, scratch = None, 0, []
+        for line in text.splitlines() + ["0 <end>:"]:
+            m = FUNCTION.match(line)
+            if m:
+                if name and "11gemm_kernel" in name:
+                    seen += 1
+                    n = sum(0 < at < mfmas for at in scratch)
+                    if n:
+                        bad[name] = n
+                name, mfmas, scratch = m.group(1), 0, []
+            elif "v_mfma" in line:
+                mfmas += 1
+            elif "scratch_" in line:
+                scratch.append(mfmas)
+    assert seen > 100, seen
     assert not bad, bad

@@ -50,9 +50,10 @@ constexpr int epi_chunk(int ntl, int ew, int nw, int ring_bytes) {
 template <int BM_, int BN_, int WGM_, int WGN_, int NST_, int OCC_, int LOOP_ = 0>
 struct GemmCfg {
   static constexpr int BM = BM_, BN = BN_, WGM = WGM_, WGN = WGN_, NST = NST_, OCC = OCC_;
-  // main loop: 0 split k-step pipeline; 2 two stages per barrier, the operands read half a stage ahead;
-  // 3 128-byte stages, loader waves, the operands read a whole stage ahead; 4 ping-pong (two wave groups) over
-  // 128-byte stages in two slots; 5 whole-stage operand sets, 128-byte stages in two slots
+  // main loop: 0 split k-step pipeline; 1 ping-pong (two wave groups) over 64-byte stages; 2 two stages per
+  // barrier, the operands read half a stage ahead; 3 128-byte stages, loader waves, the operands read a whole
+  // stage ahead; 4 ping-pong over 128-byte stages in two slots; 5 whole-stage operand sets, 128-byte stages in
+  // two slots
   static constexpr int LOOP = LOOP_;
   static constexpr int NW = WGM * WGN;                    // compute waves
   static constexpr int LW = LOOP == 3 ? NW : 0;           // loader waves
@@ -62,27 +63,27 @@ struct GemmCfg {
   static constexpr int BKB = stage_kb(LOOP);
   static constexpr int A_BYTES = BM * BKB, ST_BYTES = (BM + BN) * BKB;
   // a stage is NL blocks of RPB rows x BKB bytes (1 KB, one async-load instruction): A blocks 0 .. NA-1,
-  // then B blocks; block b is loaded by wave b % NW, Q blocks per wave.
+  // then B blocks; block b is loaded by wave b % NW.  Waves w < NL % NW load QH blocks, the rest QL.
   static constexpr int RPB = 1024 / BKB, CPR = BKB / 16;   // rows per block, 16-byte chunks per row
   static constexpr int NA = BM / RPB, NL = (BM + BN) / RPB;
-  static constexpr int Q = NL / NW;
+  static constexpr int QL = NL / NW, QH = (NL + NW - 1) / NW, NQH = NL % NW == 0 ? NW : NL % NW;
   static constexpr int EW = WN % 64 == 0 ? 64 : 32;       // epilogue pass width (columns)
   static constexpr int ECH = epi_chunk(NTL, EW, NW, NST * ST_BYTES);   // 32-column tiles per staging chunk
   static constexpr int NECH = (NTL + ECH - 1) / ECH;
   static constexpr int EROW = ECH * 32 * 4 + 16;          // epilogue LDS row (f32 + pad)
   static_assert(BM % RPB == 0 && BN % RPB == 0 && NA % NW == 0, "load split: A blocks evenly over the waves");
   static_assert(LOOP != 4 || (NW == 8 && NST == 2), "two-slot ping-pong: two groups of four waves");
-  static_assert(NL % NW == 0, "the same load count on every wave");
+  static_assert(LOOP == 1 || NL % NW == 0, "the same load count on every wave");
   static_assert(NW * 32 * EROW <= NST * ST_BYTES, "epilogue staging fits in the ring");
   static_assert(WN % 32 == 0, "wave tile width");
-  // ping-pong: waves w and w + 4 share a SIMD and belong to groups 0 and 1; each group loads a uniform
-  // number of blocks per stage
+  static_assert(LOOP != 1 || (NW == 8 && NST >= 3 && NQH % 4 == 0),
+                "four-slot ping-pong: two groups of four waves, uniform loads in each, two stages in flight");
   static_assert(LOOP != 2 || NST >= 5, "two-stage loop: stages it + 2, it + 3 land while it + 4 .. are in flight");
   static_assert(LOOP != 3 || NST >= 3, "whole-stage loop: two stages in flight");
   // Lean addressing for ping-pong tiles whose accumulators and three operand sets nearly fill the 256
   // registers of a wave: the async-load lane offsets that follow from others are recomputed where
   // they are used instead of being held through the main loop (held, they spilled into the loop).
-  static constexpr bool LEAN = LOOP == 4 && 16 * MT * NTL + 12 * (MT + NTL) > 190;
+  static constexpr bool LEAN = (LOOP == 1 || LOOP == 4) && 16 * MT * NTL + 12 * (MT + NTL) > (LOOP == 4 ? 190 : 232);
 };
 // 256x128 block, 128x64 per wave, two workgroups per CU
 using CfgM = GemmCfg<256, 128, 2, 2, 3, 2>;
@@ -98,6 +99,14 @@ using CfgN = GemmCfg<256, 192, 4, 2, 2, 1, 4>;
 // 256x320 block, 8 waves of 64x160: N = 2560 (the QKV projection at hd 128) in 8 column tiles, one round
 // of 256 CUs at M = 8192 where 256x192 tiles take 1.75 rounds; its epilogue stages 128 + 32 columns
 using CfgW = GemmCfg<256, 320, 4, 2, 2, 1, 4>;
+// The 256x320 block on 64-byte stages in a four-slot ring, three operand sets: for bf16, and for int8 where K is not
+// whole cache lines.  The two operand sets of the other read each half-stage's second k-step in the phase that uses
+// it, which costs bf16 more than whole lines save (us, two slots then four: f32 residual, N = 1536, K = 4608,
+// M = 10923 150, 138, M = 12000 152, 144; N = 2048, K = 6144, M = 9000 195.5, 191.5; bf16 out, N = 2560, K = 1536,
+// M = 7000 56.5, 53.5, M = 8192 57.8, 58.1, K = 2048 72.3, 73.4) and int8 once no lines are saved (N = 2560,
+// M = 8192, K = 2112 49.5, 47.6, K = 6208 118.5, 114.8; whole lines, K = 1536 36.5, 36.8, the loop before 38.2).
+// 256x256 and 256x192, with three operand sets in either loop, gain 1 - 5 % from two slots at any K.
+using CfgW4 = GemmCfg<256, 320, 4, 2, 4, 1, 1>;
 // Short problems (few tiles, each K loop latency-bound): 8-stage rings, seven stages of loads in flight.
 // 64x128 block, 32x64 per wave, one workgroup per CU (the 64x128 tile runs two stages per barrier: its waves
 // have few MFMAs per stage to cover a barrier)
@@ -231,8 +240,9 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
   const int m0 = (first_m + wig % gsz) * C::BM, n0 = (wig / gsz) * C::BN;
   const int lda = g.lda * T::ESZ, ldb = g.ldb * T::ESZ;   // bytes
   const int Kb = g.K * T::ESZ;
-  constexpr int Q = C::Q;   // async-load instructions per wave per stage
-
+  // async-load instructions per wave per stage: QH on waves w < NQH (ping-pong group 0 when uneven)
+  constexpr int Q = C::QH;
+  const bool qfull = C::QH == C::QL || w < C::NQH;
 
   // this lane's async-load sources: block b = w + NW j, rows RPB (b or b - NA) + lane / CPR of A or B, as
   // 32-bit byte offsets from the operand base (the base and the K offset stay scalar); rows past M / N
@@ -281,9 +291,9 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
   auto issue1 = [&](int j, int st, int kb) {
     char* dst = smem + st * C::ST_BYTES + (lw + C::NW * j) * 1024;
     if (j < JA) copy16_to_lds(rA, voff(j), (uint32_t)kb, dst);
-    else copy16_to_lds(rB, voff(j), (uint32_t)kb, dst);
+    else if (j < C::QL || qfull) copy16_to_lds(rB, voff(j), (uint32_t)kb, dst);
   };
-  // A last stage of half the K bytes (LOOP 4): the lanes of its other half read nothing.  The rows of a lane's
+  // A last stage of half the K bytes (HALF): the lanes of its other half read nothing.  The rows of a lane's
   // loads are multiples of 16 apart, so they share one swizzle; the K offset goes where the range check sees it.
   auto issue_half = [&](int j, int st, int kb) {
     static_assert(C::LOOP != 4 || (C::RPB * C::NW % 16 == 0 && C::BM % 16 == 0), "one swizzle per lane");
@@ -293,8 +303,9 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
   // wait until at most `n` stages of this wave's async loads are outstanding
   auto wait_stages = [&](auto nc) {
     constexpr int n = decltype(nc)::value;
-    static_assert(n * Q <= 63, "vmcnt counts at most 63 loads");
-    MK_WAIT_VMCNT(n * Q);
+    static_assert(n * C::QH <= 63, "vmcnt counts at most 63 loads");
+    if (C::QH == C::QL || qfull) MK_WAIT_VMCNT(n * C::QH);
+    else MK_WAIT_VMCNT(n * C::QL);
   };
   using W0 = std::integral_constant<int, 0>;
   // wait until at most min(n, left) stages are outstanding (left: stages there are beyond the one waited for)
@@ -391,7 +402,9 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
   constexpr bool EARLY_SCALES = C::MT * NTASK + NSB * (SILU ? 16 : 8) <= 32;
   if (EARLY_SCALES && dq && !loader) load_scales();
 
-  const int nk = C::LOOP == 4 ? (Kb + BKB - 1) / BKB : Kb / BKB;   // stages
+  // the last stage may hold half the K bytes (256x320: taken for whole ones only)
+  constexpr bool HALF = C::LOOP == 4 && BN != 320;
+  const int nk = HALF ? (Kb + BKB - 1) / BKB : Kb / BKB;   // stages
   // stages loaded ahead of the main loop: NST - 1 (NST - 2 for the two-stage loop, whose iterations
   // load two stages each; stages 0 and 1 visible after the barrier there, stage 0 in the others)
   // (every slot for the whole-stage loop); stages 0 and 1 visible after the barrier
@@ -399,7 +412,7 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
   if (C::LW == 0 || loader) {
 #pragma unroll
     for (int s0 = 0; s0 < PRE; ++s0)
-      if (C::LOOP == 4 && s0 < nk && (s0 + 1) * BKB > Kb) {
+      if (HALF && s0 < nk && (s0 + 1) * BKB > Kb) {
 #pragma unroll
         for (int j = 0; j < Q; ++j) issue_half(j, s0, s0 * BKB);
       } else if (s0 < nk) {
@@ -414,7 +427,106 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
   // Materialize the epilogue's kernel arguments now: a scalar load still pending inside the loop would
   // turn every LDS wait there into lgkmcnt(0) (scalar loads return out of order).
   asm volatile("" ::"s"(g.out), "s"(g.res), "s"(g.rs), "s"(g.cs), "s"(g.aux), "s"(g.ldo), "s"(g.ldr));
-  if constexpr (C::LOOP == 4) {
+  if constexpr (C::LOOP == 1) {
+    // Ping-pong.  The waves form two groups (wm = 0, 1) with one wave of each on every SIMD, and each
+    // iteration is a memory phase M (async loads of the stage NST - 1 ahead) and a compute phase C
+    // (the stage's MFMAs, with the next stage's operands read from LDS into registers alongside), each
+    // closed by a barrier.  Group 1 starts one barrier late, so on every SIMD one wave issues MFMAs
+    // while the other is in its memory phase or waiting at the barrier.
+    // Operands live in a ring of three k-step register sets: stage s uses (2s, 2s + 1) mod 3, and
+    // stage s + 1's k-step 0 goes to the free set, its k-step 1 to the set stage s's k-step 0 used.
+    // Stage s + 1 must be visible when group 0 starts C(s): group 0 waits for its loads of stage s + 1
+    // at the end of M(s), group 1 at the end of C(s - 1).  A stage's slot is refilled in M(s + 1) of
+    // the stage NST ahead, after both groups finished reading it in their C(s - 1).
+    constexpr int D = C::NST - 1;
+    constexpr int NOP = C::MT + C::NTL;                   // operand registers per k-step: B then A
+    u32x4 H0[NOP], H1[NOP], H2[NOP];
+    static_assert(!T::WIDE, "one k-step per operand set");
+    auto rdq = [&](const char* Sb, int ks, int q, u32x4 (&dst)[NOP]) {
+      if (q < C::NTL) dst[q] = *reinterpret_cast<const u32x4*>(Sb + (ks ? bo1 : bo0) + q * 32 * BKB);
+      else dst[q] = *reinterpret_cast<const u32x4*>(Sb + (ks ? ao1 : ao0) + (q - C::NTL) * 32 * BKB);
+    };
+    auto mfq = [&](int i, const u32x4 (&src)[NOP]) {
+      const int mt = i / C::NTL, nt = i % C::NTL;
+      acc[mt][nt] = T::run(src[C::NTL + mt], src[nt], acc[mt][nt]);
+    };
+    // stages 0 and 1 visible; stage 0 in H0 / H1
+    if (nk >= D) wait_stages(std::integral_constant<int, D - 2>{});
+    else wait_stages(W0{});
+    lds_barrier();
+#pragma unroll
+    for (int q = 0; q < NOP; ++q) rdq(smem, 0, q, H0);
+#pragma unroll
+    for (int q = 0; q < NOP; ++q) rdq(smem, 1, q, H1);
+    __builtin_amdgcn_s_waitcnt(0xc07f);
+    // ping-pong group of this wave: waves w and w + 4 share a SIMD; group 0 loads QH blocks per stage,
+    // group 1 QL
+    const int wgrp = w >> 2;
+    if (wgrp == 1) lds_barrier();
+    int cur = 0;
+    // `steady` instances (stage it + D exists) have no runtime conditions, so the compute phase stays one
+    // basic block instead of a branch around every operand read
+    auto step = [&](auto steady, int it, u32x4 (&ha)[NOP], u32x4 (&hb)[NOP], u32x4 (&hc)[NOP]) {
+      constexpr bool ST = decltype(steady)::value;
+      // M(it): async loads of stage it + D into the slot of stage it - 1
+      const bool pre = ST || it + D < nk;
+      if (pre) {
+        const int nslot = cur == 0 ? C::NST - 1 : cur - 1;
+#pragma unroll
+        for (int j = 0; j < Q; ++j) issue1(j, nslot, (it + D) * BKB);
+      }
+      if (wgrp == 0 && (ST || it + 1 < nk)) {
+        if (pre) MK_WAIT_VMCNT((D - 1) * C::QH);
+        else MK_WAIT_VMCNT(0);
+      }
+      lds_barrier();
+      // C(it): MFMAs of stage it, reads of stage it + 1
+      const int s1 = cur == C::NST - 1 ? 0 : cur + 1;
+      const char* S1 = smem + s1 * C::ST_BYTES;
+      const bool nxt = ST || it + 1 < nk;
+      __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+      for (int i = 0; i < NMF; ++i) {
+        mfq(i, ha);
+        if (i < NOP && nxt) rdq(S1, 0, i, hc);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int q = NMF; q < NOP; ++q)
+        if (nxt) rdq(S1, 0, q, hc);
+#pragma unroll
+      for (int i = 0; i < NMF; ++i) {
+        mfq(i, hb);
+        if (i < NOP && nxt) rdq(S1, 1, i, ha);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+#pragma unroll
+      for (int q = NMF; q < NOP; ++q)
+        if (nxt) rdq(S1, 1, q, ha);
+      __builtin_amdgcn_s_setprio(0);
+      __builtin_amdgcn_s_waitcnt(0xc07f);                 // lgkmcnt(0): stage it + 1 is in registers
+      if (wgrp == 1 && (ST || it + 2 < nk)) {
+        if (pre) MK_WAIT_VMCNT((D - 2) * C::QL);
+        else MK_WAIT_VMCNT(0);
+      }
+      lds_barrier();
+      cur = s1;
+    };
+    using Steady = std::integral_constant<bool, true>;
+    using Tail = std::integral_constant<bool, false>;
+    int it = 0;
+    for (; it + 2 + D < nk; it += 3) {
+      step(Steady{}, it, H0, H1, H2);
+      step(Steady{}, it + 1, H2, H0, H1);
+      step(Steady{}, it + 2, H1, H2, H0);
+    }
+    for (; it < nk; it += 3) {
+      step(Tail{}, it, H0, H1, H2);
+      if (it + 1 < nk) step(Tail{}, it + 1, H2, H0, H1);
+      if (it + 2 < nk) step(Tail{}, it + 2, H1, H2, H0);
+    }
+    if (wgrp == 0) lds_barrier();
+  } else if constexpr (C::LOOP == 4) {
     // Ping-pong over 128-byte stages in two LDS slots: whole cache lines per row, two half-stages (64 bytes of
     // K) of MFMAs per stage.  With 64-byte slices every load of a line's other half, a stage later, misses
     // the 32 KB L1 again and L2 delivers each line twice.
@@ -503,7 +615,7 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
       if (p < nfull) {
 #pragma unroll
         for (int j = 0; j < Q; ++j) issue1(j, p & 1, p * BKB);
-      } else if (p < nk) {
+      } else if (HALF && p < nk) {
 #pragma unroll
         for (int j = 0; j < Q; ++j) issue_half(j, p & 1, p * BKB);
       }
@@ -1423,6 +1535,18 @@ template <> struct TileOf<11> { using C = CfgH; };
 template <> struct TileOf<12> { using C = CfgP; };
 template <> struct TileOf<13> { using C = CfgQ; };
 
+template <int ID, GemmIn IN, Epi EPI>
+void launch_id(const GemmArgs& g, hipStream_t st) {
+  if constexpr (ID == 8 && IN == GemmIn::BF16) {
+    launch_c<CfgW4, IN, EPI>(g, st);
+  } else {
+    if constexpr (ID == 8) {
+      if (g.K * Mma<IN>::ESZ % 128) return launch_c<CfgW4, IN, EPI>(g, st);
+    }
+    launch_c<typename TileOf<ID>::C, IN, EPI>(g, st);
+  }
+}
+
 template <GemmIn IN, Epi EPI>
 int launch_t(const GemmArgs& g, hipStream_t st) {
   constexpr bool silu = EPI == Epi::DQ_SILU || EPI == Epi::DQ_SILU_F32A || EPI == Epi::SILU_BF16;
@@ -1430,7 +1554,7 @@ int launch_t(const GemmArgs& g, hipStream_t st) {
 #define MK_TILE(ID)                                          \
   if constexpr (gemm_tile_built(ID, silu, IN)) {             \
     if (id == ID) {                                          \
-      launch_c<typename TileOf<ID>::C, IN, EPI>(g, st);      \
+      launch_id<ID, IN, EPI>(g, st);                         \
       return MK_OK;                                          \
     }                                                        \
   }

@@ -340,9 +340,10 @@ def test_gate_up_tiles_match(M, N, K):
 @pytest.mark.parametrize("N", [1536, 2048, 2560])
 @pytest.mark.parametrize("kb", [64, 128, 192, 384, 448, 1600, 4160])
 def test_gemm_ping_pong_stages(N, kb):
-    """256x192, 256x256 and 256x320 (bf16, int8) ping-pong tiles (M = 8100, ragged): K of one half-stage up to 65, whole and half last
-    stages, over every remainder of the unrolled loop: int8 exact, bf16 within 64 eps sum|products| of
-    float64, fp8 within 1e-4 sum|products| (the fp8 unit's own precision)."""
+    """256x192, 256x256 and 256x320 (bf16, int8) ping-pong tiles (M = 8100, ragged): K of 64 bytes up to 65 times
+    that, over every remainder of the unrolled loops, on 128-byte stages with whole and half last ones and (256x320
+    in bf16 and with half lines of K) on 64-byte stages: int8 exact, bf16 within 64 eps sum|products| of float64, fp8 within 1e-4 sum|products| (the fp8
+    unit's own precision)."""
     from minicpm5_mk import ops
 
     dev = _dev()
@@ -361,10 +362,11 @@ def test_gemm_ping_pong_stages(N, kb):
     assert (err <= 1e-4 * (af.double().abs() @ bf.double().abs().t())).all()
 
 
+@pytest.mark.parametrize("fp8", [False, True])
 @pytest.mark.parametrize("N", [1536, 2048, 2560])
-@pytest.mark.parametrize("K", [32, 96, 800])
-def test_gemm_operand_column_range(N, K):
-    """bf16 operands that are the last K columns of wider matrices (row stride K + 40, the last row ends with the
+@pytest.mark.parametrize("kb", [64, 192, 1600])
+def test_gemm_operand_column_range(N, kb, fp8):
+    """Operands that are the last columns of wider matrices (row stride K + 80 bytes, the last row ends with the
     allocation), K bytes an odd multiple of 64: the ping-pong tiles' half stage stops at K, f32 bits equal to those
     of contiguous copies."""
     import ctypes
@@ -372,15 +374,17 @@ def test_gemm_operand_column_range(N, K):
     from minicpm5_mk import _lib, ops
 
     dev = _dev()
-    g = torch.Generator().manual_seed(N + K)
-    M, ld = 8100, K + 40
-    print(f"[column range] {M}x{N}x{K}", flush=True)
-    a = torch.randn(M, ld, generator=g).to(BF16).to(dev)[:, 40:]
-    b = torch.randn(N, ld, generator=g).to(BF16).to(dev)[:, 40:]
+    g = torch.Generator().manual_seed(N + kb)
+    dt, esz = (torch.float8_e4m3fn, 1) if fp8 else (BF16, 2)
+    M, K, pad = 8100, kb // esz, 80 // esz
+    ld = K + pad
+    print(f"[column range] {M}x{N} K bytes {kb} {dt}", flush=True)
+    a = torch.randn(M, ld, generator=g).to(dt).to(dev)[:, pad:]
+    b = torch.randn(N, ld, generator=g).to(dt).to(dev)[:, pad:]
     out = torch.empty(M, N, dtype=torch.float32, device=dev)
     ptr = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
-    _lib.check(_lib.load().mk_gemm(0, _lib.EPI["f32"], ptr(a), ld, ptr(b), ld, M, N, K, ptr(out), N, None, 0, None, None,
-                                   None, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "mk_gemm")
+    _lib.check(_lib.load().mk_gemm(2 if fp8 else 0, _lib.EPI["f32"], ptr(a), ld, ptr(b), ld, M, N, K, ptr(out), N, None,
+                                   0, None, None, None, ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)), "mk_gemm")
     ref = ops.gemm(a.contiguous(), b.contiguous(), "f32")
     assert torch.equal(out.view(torch.int32), ref.view(torch.int32))
 

@@ -592,14 +592,16 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
     auto pf_row = [&](int l) {
       return w == 0 ? (uint32_t)min(pm + l, g.M - 1) * (uint32_t)lda : (uint32_t)min(pn + l, g.N - 1) * (uint32_t)ldb;
     };
-    const uint32_t pfo = LEAN ? 0 : pf_row(lane);
+    // Held through the loop, the offset was spilled by the fp8 256x256 instances with SiLU or residual epilogues,
+    // and its reload, behind the stage's loads, waited for all of them.  They derive it from the lane number at
+    // each use: 2B gate/up at M = 4096 114 us, now 102, at M = 8192 204, now 191.  Where it fits it is held: the
+    // short fp8 loops without an epilogue to spill for take 4 - 7 % longer otherwise (QKV, M = 12000 58, 62 us).
+    constexpr bool DERIVE = LEAN && T::WIDE && (SILU || RES);
+    const uint32_t pfo = DERIVE ? 0 : pf_row(lane);
     auto prefetch = [&](int p) {
       if (!pfw || p >= nk) return;
       uint32_t o = pfo;
-      if constexpr (LEAN) {
-        // lean addressing: from the lane number, at each use.  Held, the offset was spilled in the fp8 256x256
-        // SiLU instance, and its reload, behind the stage's loads, waited for all of them: 2B gate/up at
-        // M = 4096 114 us, now 99, at M = 8192 204, now 190.
+      if constexpr (DERIVE) {
         uint32_t ones = ~0u;
         asm volatile("" : "+s"(ones));
         o = pf_row((int)__builtin_amdgcn_mbcnt_hi(ones, __builtin_amdgcn_mbcnt_lo(ones, 0)));

@@ -63,6 +63,9 @@ inline int gemm_tile(bool silu, GemmIn in, int M, int N, int kb) {
     // 192x128 pairs fill rounds the larger tiles leave half empty: 2B gate/up at M = 1536 52.0 -> 43.9 us, at
     // M = 3072 88.4 -> 82.6, 1B gate/up at M = 6000 103 -> 96.7
     if (o.id == 12 && !line) continue;
+    // but alone on its CU, three rows of int8 tiles lose to two of 256x128: 1B gate/up at M = 400 15.3 us, now 14.8
+    // (M = 576, three rows either way, 15.1 against 16.6; bf16 24.0 against 27.2)
+    if (o.id == 12 && in == GemmIn::I8 && fits(192, 128) && M > 384 && M <= 512) continue;
     const long rounds = (tiles(o.bm, o.bn) + 255) / 256;
     const double t = (double)rounds * o.bm * o.bn / o.eff;
     if (t < bt * 0.999) {

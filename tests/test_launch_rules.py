@@ -111,3 +111,9 @@ def test_gemm_tile_is_built(rules):
                         t = rules.gemm_tile(silu, in_type, M, N, kb)
                         assert rules.gemm_tile_built(t, silu, in_type), (silu, in_type, M, N, kb, t)
                         assert kb % 128 == 0 or not (t == 6 or t >= 9), (silu, in_type, M, N, kb, t)
+
+
+def test_gate_up_tile_of_two_rows(rules):
+    """int8 gate/up of 385 .. 512 rows: two rows of 256x128 tiles, not three of 192x128, one workgroup per CU."""
+    assert [rules.gemm_tile(1, I8, m, 9216, 1536) for m in (384, 385, 400, 512, 513)] == [3, 2, 2, 2, 12]
+    assert rules.gemm_tile(1, I8, 3072, 1536, 256) == 12

@@ -13,10 +13,10 @@
   * activation quantisation in the fp8d / int8 / fp8 modes: bit-exact codes (the static modes with
     RMSNorm round x * rstd to bf16, so an rstd one f32 ulp off may move a code by one step: at most
     0.1% of codes, each by one step); f32 -> e4m3 conversion bit-exact over every finite bf16 value.
-  * fp8 GEMM: the fp8 MFMAs (v_mfma_f32_32x32x64_f8f6f4) sum their products at reduced internal precision (measured
-    on MI355X: max error 2.4e-5 of sum|products| at K = 64, 1.5e-6 at K = 4608, zero when the products
-    span few binades), so the bound is 1e-4 * sum|products| of the exact (float64) result; dequant
-    epilogues within 1 bf16 ulp + that bound.
+  * fp8 GEMM: the fp8 MFMAs sum their products at reduced internal precision.  Measured on MI355X with
+    v_mfma_f32_32x32x64_f8f6f4 (the K = 16 instructions give the same): max error 6.2e-5 of sum|products| at
+    K = 64, 1.2e-5 at K = 448, 2.2e-6 at K = 4608, 1.5e-5 in 2-norm at every K.  So the bound is
+    1e-4 * sum|products| of the exact (float64) result; dequant epilogues within 1 bf16 ulp + that bound.
 """
 import math
 
@@ -194,8 +194,8 @@ def test_row_quant_scale_tree_bitexact(T, H):
 @pytest.mark.parametrize("M,N,K", [(256, 128, 64), (300, 200, 1536), (8192, 1920, 1536), (8192, 2560, 1536),
                                    (1000, 1536, 4608), (1000, 1536, 1088)])
 def test_gemm_int8_exact(M, N, K):
-    """Exact int32 products; (8192, 1920) and (8192, 2560) (the QKV projections at hd 96 and 128) take the
-    256x320 tile, whose epilogue stages its 64x160 wave tiles in two column chunks."""
+    """Exact int32 products; (8192, 1920) and (8192, 2560) are the QKV projections at hd 96 and 128, on the
+    256x256 and on the 256x320 tile, whose epilogue stages its 64x160 wave tiles in two column chunks."""
     from minicpm5_mk import ops
     from oracle import emulate
 
@@ -257,9 +257,9 @@ def test_gemm_bf16(M, N, K):
 
 @pytest.mark.parametrize("N,K", [(1536, 4608), (1536, 2080), (1536, 544)])
 def test_gemm_bf16_rows_independent_of_tile(N, K):
-    """The first 1000 rows of a 4096-row product take the 64x128 short-problem tile (its two-stage loop;
-    odd stage counts at K = 2080 and at K = 544, 17 stages, the fewest it is chosen for) alone and a wide
-    tile inside the big product: identical f32 bits."""
+    """The first 1000 rows of a 4096-row product alone, on a 64x128 tile (loader waves at K = 4608, the two-stage
+    loop with an odd stage count at K = 2080 and at K = 544, 17 stages, the fewest it is chosen for), and on
+    128x128 pairs or 256x128 tiles inside the big product: identical f32 bits."""
     from minicpm5_mk import ops
 
     dev = _dev()
@@ -337,6 +337,67 @@ def test_gate_up_tiles_match(M, N, K):
     assert torch.equal(out.view(torch.int16), big[:M].view(torch.int16))
 
 
+# (tile configuration, M, N, K bytes): the tile is checked against the dispatch rule on the CPU (test_launch_rules)
+TILE_SHAPES = [
+    (10, 33, 72, 128), (10, 250, 1504, 4608), (9, 321, 1528, 256), (9, 500, 1504, 640), (11, 1000, 1512, 4224),
+    (6, 2000, 1512, 4224), (13, 2300, 2008, 384), (7, 512, 2560, 1024), (7, 512, 2560, 1088), (7, 512, 2560, 1536),
+    (3, 1500, 1528, 128), (3, 1500, 1528, 192), (3, 1500, 1528, 256), (3, 1500, 1528, 960), (2, 40000, 128, 192),
+    (2, 40000, 128, 320)]
+
+
+@pytest.mark.parametrize("tile,M,N,kb", TILE_SHAPES)
+def test_gemm_every_tile(tile, M, N, kb):
+    """Every tile below the ping-pong ones, each loop with one stage, fewer stages than ring slots, odd, even and many
+    (fp8 takes a stage in one wide k-step, so its loops differ): fp8 and bf16 bits equal to the same rows of a
+    product of 9000 rows, fp8 within 1e-4 and bf16 within 64 eps of sum|products| of float64, int8 exact."""
+    from minicpm5_mk import ops
+
+    dev = _dev()
+    g = torch.Generator().manual_seed(M + N + kb)
+    rows = max(M, 9000)
+    print(f"[tile {tile}] {M}x{N} K bytes {kb}", flush=True)
+
+    def same(a, b):
+        out, other = ops.gemm(a[:M].contiguous(), b, "f32"), ops.gemm(a[:9000].contiguous(), b, "f32")
+        n = min(M, 9000)
+        assert torch.equal(out[:n].view(torch.int32), other[:n].view(torch.int32))
+        return out.double(), a[:M].double() @ b.double().t(), a[:M].double().abs() @ b.double().abs().t()
+
+    out, ref, mag = same(*(t.to(dev) for t in _fp8_pair(rows, N, kb, 7)))
+    assert ((out - ref).abs() <= 1e-4 * mag).all()
+    a = torch.randn(rows, kb // 2, generator=g).to(BF16).to(dev)
+    b = (torch.randn(N, kb // 2, generator=g) * 0.02).to(BF16).to(dev)
+    out, ref, mag = same(a, b)
+    assert ((out - ref).abs() <= 64 * 2.0 ** -24 * mag).all()
+    ai = torch.randint(-127, 128, (M, kb), generator=g, dtype=torch.int8).to(dev)
+    bi = torch.randint(-127, 128, (N, kb), generator=g, dtype=torch.int8).to(dev)
+    assert torch.equal(ops.gemm(ai, bi, "i32").double(), ai.double() @ bi.double().t())
+
+
+SILU_SHAPES = [(7, 100, 9216, 1536), (3, 200, 9216, 1536), (12, 576, 9216, 1536), (12, 1500, 12288, 256),
+               (12, 1400, 12288, 128), (12, 5990, 9216, 384), (4, 1792, 9216, 1536)]
+
+
+@pytest.mark.parametrize("tile,M,N,kb", SILU_SHAPES)
+def test_gate_up_tiles_match_float(tile, M, N, kb):
+    """SILU_BF16 with fp8 operands (dequantised) and with bf16 ones on each gate/up tile: rows bitwise equal to the
+    same rows of a product of 8192."""
+    from minicpm5_mk import ops
+
+    dev = _dev()
+    g = torch.Generator().manual_seed(M + N + kb)
+    print(f"[gate/up tile {tile}] {M}x{N} K bytes {kb}", flush=True)
+    a, b = (t.to(dev) for t in _fp8_pair(8192, N, kb, 8))
+    rs, cs = (torch.rand(8192, generator=g) * 1e-3).to(dev), (torch.rand(N, generator=g) * 1e-3).to(dev)
+    big = ops.gemm(a, b, "silu_bf16", rs=rs, cs=cs)
+    out = ops.gemm(a[:M].contiguous(), b, "silu_bf16", rs=rs[:M].contiguous(), cs=cs)
+    assert torch.equal(out.view(torch.int16), big[:M].view(torch.int16))
+    a = torch.randn(8192, kb // 2, generator=g).to(BF16).to(dev)
+    b = (torch.randn(N, kb // 2, generator=g) * 0.1).to(BF16).to(dev)
+    big, out = ops.gemm(a, b, "silu_bf16"), ops.gemm(a[:M].contiguous(), b, "silu_bf16")
+    assert torch.equal(out.view(torch.int16), big[:M].view(torch.int16))
+
+
 @pytest.mark.parametrize("N", [1536, 2048, 2560])
 @pytest.mark.parametrize("kb", [64, 128, 192, 384, 448, 1600, 4160])
 def test_gemm_ping_pong_stages(N, kb):
@@ -393,7 +454,7 @@ def test_gemm_operand_column_range(N, kb, fp8):
 def test_gemm_wide_tile_rows_match(epi):
     """M = 8192, N = 2560 takes the 256x320 tile (one round of 256 CUs; 64x160 wave tiles, the epilogue
     staged in a 128- and a 32-column chunk, the offsets of later async loads recomputed per load), M = 1000
-    the 256x192 one: the first 1000 rows are bitwise equal for each epilogue, and the f32 products match
+    the 128x128 one: the first 1000 rows are bitwise equal for each epilogue, and the f32 products match
     a float64 reference on rows at both ends."""
     from minicpm5_mk import ops
 

@@ -615,11 +615,14 @@ def test_forward_timed_matches_forward():
 
 @pytest.mark.parametrize("name,quant,B,S", [
     ("tiny", "int8d:qkv+gu|sq|lastbf16|fqkv|fmlp", 2, 512), ("tiny-hd96", "int8d:qkv+gu+o|sq|lastbf16", 3, 256),
-    ("tiny", "bf16", 2, 384), ("tiny-hd96", "fp8d|sq|lastbf16", 1, 640), ("tiny", "int8|sq|fqkv|fmlp", 2, 256)])
+    ("tiny", "bf16", 2, 384), ("tiny-hd96", "fp8d|sq|lastbf16", 1, 640), ("tiny", "int8|sq|fqkv|fmlp", 2, 256),
+    ("tiny", "int8d:qkv+gu|sq|lastbf16|fqkv|fmlp", 8, 512), ("tiny", "bf16", 4, 1024),
+    ("tiny-hd96", "fp8d|sq|lastbf16", 9, 256)])
 def test_fused_attn_prep_equals_prep_kernel(name, quant, B, S):
     """The QKV projection's routing epilogue (K RoPE'd into krope, V transposed into vt, pack.hip map 2
     column order) gives the same model output, bitwise, as the projection followed by the separate prep
-    kernel, for every QKV epilogue (DQ_BF16, DQ2_BF16, BF16, fp8 DQ2_BF16) and both head dims."""
+    kernel, for every QKV epilogue (DQ_BF16, DQ2_BF16, BF16, fp8 DQ2_BF16) and both head dims, on the tiles of
+    short prompts and, from 2304 tokens on, on the 128x128 pairs."""
     from minicpm5_mk.config import preset
     from minicpm5_mk.synth import random_hf_state_dict, random_token_ids
 

@@ -117,3 +117,24 @@ def test_gate_up_tile_of_two_rows(rules):
     """int8 gate/up of 385 .. 512 rows: two rows of 256x128 tiles, not three of 192x128, one workgroup per CU."""
     assert [rules.gemm_tile(1, I8, m, 9216, 1536) for m in (384, 385, 400, 512, 513)] == [3, 2, 2, 2, 12]
     assert rules.gemm_tile(1, I8, 3072, 1536, 256) == 12
+
+
+def test_gemm_tile_of_tested_shapes(rules):
+    """The GPU tests reach the tiles that they name."""
+    from test_gpu_kernels import SILU_SHAPES, TILE_SHAPES
+
+    for t, M, N, kb in TILE_SHAPES:
+        assert [rules.gemm_tile(0, i, M, N, kb) for i in (I8, BF16, F8)] == [t] * 3, (t, M, N, kb)
+    for t, M, N, kb in SILU_SHAPES:
+        assert [rules.gemm_tile(1, i, M, N, kb) for i in (BF16, F8)] == [t] * 2, (t, M, N, kb)
+    assert {t for t, *_ in TILE_SHAPES} == {2, 3, 6, 7, 9, 10, 11, 13} and {t for t, *_ in SILU_SHAPES} == {3, 4, 7, 12}
+    # ping-pong stages and the routed QKV projection of the model tests (N = 1280 and 1920)
+    for N, t in ((1536, 5), (2048, 4), (2560, 8)):
+        for kb in (64, 128, 192, 384, 448, 1600, 4160):
+            assert [rules.gemm_tile(0, i, 8100, N, kb) for i in (I8, BF16)] == [t] * 2, (N, kb)
+    assert rules.gemm_tile(0, F8, 8100, 2560, 192) == 5
+    assert rules.gemm_tile(0, I8, 8192, 1920, 1536) == 4 and rules.gemm_tile(0, I8, 8192, 2560, 1536) == 8
+    assert [rules.gemm_tile(0, BF16, 1000, 1536, 2 * k) for k in (4608, 2080, 544)] == [11, 7, 7]
+    assert [rules.gemm_tile(0, BF16, 4096, 1536, 2 * k) for k in (4608, 2080, 544)] == [13, 2, 2]
+    assert rules.gemm_tile(0, I8, 4096, 1280, 256) == 13 and rules.gemm_tile(0, BF16, 4096, 1280, 512) == 13
+    assert rules.gemm_tile(0, F8, 2304, 1920, 384) == 13

@@ -8,8 +8,8 @@
 // accumulation) and fp8 e4m3 (v_mfma_f32_32x32x64_f8f6f4, f32 accumulation) share one kernel: int8 and bf16
 // consume 16 bytes of K per lane per MFMA, fp8 32 (the whole 64-byte stage slice in one k-step, at twice
 // the rate of the K = 16 fp8 instruction; against float64 its sums are off by the same 1.5e-5 in 2-norm and
-// 1.5 - 3.8e-6 of sum|products| at K = 1536 .. 6144, M = 64 .. 4096).  2B gate/up at M = 4096: 144 -> 103 us,
-// QKV 39 -> 29 us.
+// 1.9 - 4.7e-6 of sum|products| at K = 1536 .. 6144, M = 64 .. 4096).  2B gate/up at M = 4096 152 us with the
+// K = 16 instruction, 102 now; QKV at M = 8192 48, 40.
 //
 // Epilogues restate the reference's dequant / activation / residual algebra exactly:
 //   fused_qkv      mk_mlp.py:169-170   out = bf16((acc * sx) * s_w)
@@ -32,7 +32,7 @@ namespace mk {
 
 namespace {
 
-// K bytes per LDS stage: 64 (two MFMA k-steps); 128 (four, whole cache lines) in the short-problem loop
+// K bytes per LDS stage: 64 (two MFMA k-steps); 128 (four, whole cache lines) in loops 3, 4 and 5
 constexpr int stage_kb(int loop) { return loop >= 3 ? 128 : 64; }
 // threads per workgroup: the short-problem loop has as many loader waves (they only issue the async loads)
 // as compute waves
@@ -260,7 +260,7 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
       loff[j] = (uint32_t)min(n0 + r, g.N - 1) * (uint32_t)ldb + 16u * stage_chunk<BKB>(lane, r);
     }
   }
-  // Lean addressing: load j's rows are 16 NW j rows past load 0's (A) or load JA's (B), with the same
+  // Lean addressing: load j's rows are RPB NW j rows past load 0's (A) or load JA's (B), with the same
   // swizzle; the offset is clamped into the last row (rows past M / N are never stored), whose last
   // 16-byte chunk plus the largest K offset still ends inside the buffer (the range check covers the
   // lane offset only).  The empty asm keeps the sum from being hoisted out of the loop into a register
@@ -326,7 +326,7 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
     for (int j = 0; j < C::NTL; ++j) acc[i][j] = Acc{};
 
   // LDS operand reads.  Row wm WM + 32 mt + col of A has swizzle swz(col) (WM and 32 are multiples of
-  // 16), so tile mt is a fixed 2 KB step from tile 0 and the per-k-step lane offsets are two registers.
+  // 16), so tile mt is a fixed step of 32 BKB bytes from tile 0 and the per-k-step lane offsets are two registers.
   const int sw = swz<BKB>(col);
   const int aro = (wm * C::WM + col) * BKB, bro = C::A_BYTES + (wn * C::WN + col) * BKB;
   const int ao0 = aro + 16 * (half ^ sw), ao1 = aro + 16 * ((2 + half) ^ sw);
@@ -349,7 +349,7 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
     if constexpr (T::WIDE) acc[mt][nt] = mfma_fp8_32x32x64(ra0[mt], ra1[mt], rb0[nt], rb1[nt], acc[mt][nt]);
   };
 
-  // Software pipeline over the LDS ring (stage = BKB bytes of K = two MFMA k-steps):
+  // Software pipeline over the LDS ring in loop 0 (a stage is two MFMA k-steps; the others say their own):
   //   R0 / R1 hold the operands of k-step 0 / 1.  Iteration it: read k-step 1 of stage it into R1;
   //   the MFMAs of k-step 0 interleaved with the async loads of stage it + NST - 1; part of k-step 1's
   //   MFMAs; wait for stage it + 1, barrier, read its k-step 0 into R0; the rest of k-step 1's MFMAs.
@@ -405,9 +405,9 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
   // the last stage may hold half the K bytes (256x320: taken for whole ones only)
   constexpr bool HALF = C::LOOP == 4 && BN != 320;
   const int nk = HALF ? (Kb + BKB - 1) / BKB : Kb / BKB;   // stages
-  // stages loaded ahead of the main loop: NST - 1 (NST - 2 for the two-stage loop, whose iterations
-  // load two stages each; stages 0 and 1 visible after the barrier there, stage 0 in the others)
-  // (every slot for the whole-stage loop); stages 0 and 1 visible after the barrier
+  // stages loaded ahead of the main loop: every slot in the loops over 128-byte stages, else all but one
+  // (loop 2, whose iterations load two stages each: but two).  Visible after the barrier: stage 0, in loops 2
+  // and 3 stage 1 too.
   constexpr int PRE = C::LOOP >= 3 ? C::NST : C::LOOP == 2 ? C::NST - 2 : C::NST - 1;
   if (C::LW == 0 || loader) {
 #pragma unroll
@@ -536,7 +536,7 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
     // barrier late, so on every SIMD one wave issues MFMAs while the other is in its memory phase or waiting.
     // Operands live in a ring of three k-step register sets: C(h) reads half-stage h + 1's k-step 0 into the
     // free set and its k-step 1 into the set h's k-step 0 used.
-    //  Number the barrier intervals so that group 0 runs M(h) in 2h and C(h) in
+    // Number the barrier intervals so that group 0 runs M(h) in 2h and C(h) in
     // 2h + 1, group 1 M(h) in 2h + 1 and C(h) in 2h + 2.  Stage p - 1's last reads (half 2p - 1) are in
     // C(2p - 2): intervals 4p - 3 and 4p - 2, so its slot takes stage p + 1 from interval 4p - 1 on: group 1
     // loads it in M(2p - 1) (4p - 1), group 0 in M(2p) (4p).  Its first reads are group 0's C(2p + 1), interval
@@ -1247,7 +1247,7 @@ __global__ __launch_bounds__(block_threads(WGM, WGN, LOOP), OCC) void gemm_kerne
   }
 }
 
-// ---- skinny GEMM: M <= 32 (last-token layer, LM head): weight streaming.  One wave per (32 output
+// ---- skinny GEMM: M <= 32 (last-token layer, LM heads of few rows): weight streaming.  One wave per (32 output
 // columns, K range); every lane keeps SK_U k-steps of weight loads in flight (8 KB per wave) so the
 // weight stream runs near HBM rate.  With a workspace the K range is split over SK > 1 waves per
 // column block: each writes its f32 partial sums, and a second kernel adds them in split order (no

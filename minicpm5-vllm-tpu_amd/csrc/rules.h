@@ -115,9 +115,10 @@ inline bool prefetch_any(const PrefetchRanges& pf) {
 // 33.6, hd 96 20.8, 27.9; (2, 1536): hd 96 32.6, 36.8).  At hd 128 a batch of one or two long sequences has few long
 // tiles and the second items are its short ones: there 4 waves still win, with the K / V preparation, up to 15/16 of
 // the CUs for one sequence ((1, 3200) 80.1, 74.3; (1, 3584) 87.8, 84.5; (1, 3840) 94.0, 93.5; (1, 3968) 97.5, 98.5)
-// and below 3/4 for two ((2, 1216) 41.2, 39.4; (2, 1344) 44.5, 42.8; (2, 1536) 48.6, 49.9).  Inside a model the CUs that 8
-// waves leave free read the next weights, which is worth more from 3/4 of the CUs on for one sequence (2B forward:
-// (1, 3456) 13.96 ms, 14.40; (1, 3840) 15.3, 15.9) and for two (1B (2, 1280) 3.98, 4.67).
+// and below 3/4 for two ((2, 1216) 41.2, 39.4; (2, 1344) 44.5, 42.8; (2, 1536) 48.6, 49.9).  Inside a model the CUs
+// that 8 waves leave free read the next weights, which is worth more from 3/4 of the CUs on for one sequence and at
+// any size for two (forwards, ms, 8 then 4 waves: 2B (1, 3456) 13.7, 14.2, (1, 3840) 15.2, 15.9, (2, 1280) 10.6, 11.4; 1B
+// (1, 3456) 6.50, 6.48, (1, 3840) 6.53, 6.89, (2, 1280) 4.06, 4.29).
 inline int attn_waves(int items8, int ncu, int hd, int B, bool prefetch) {
   if (2 * items8 <= ncu) return 4;
   if (hd == 128 && B == 1 && 16 * items8 <= (prefetch ? 12 : 15) * ncu) return 4;
